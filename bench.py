@@ -23,6 +23,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME]
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -249,7 +250,13 @@ def run_ivfpq(args, w):
 
     K, M = p["codebook_size"], p["num_codebooks"]
     exact = args.opq or args.mode == "exact"
-    if K == 16:
+    route = ctypes.c_int(0)
+    v._lib.check(v._lib.load().vgpu_test_scan_route(ix._h, nq, k, nprobe, pool or 0, ctypes.byref(route)))
+    if route.value:
+        # the whole scan by inverted list (pairs, sample, scores, rescoring) is
+        # timed as one; list_score_kernel is its largest part
+        kernel, kname = "list_score_kernel", "scan_list"
+    elif K == 16:
         kernel, kname = "fastscan_kernel", "fastscan"
     elif exact:
         kernel, kname = f"scan8_exact_kernel<{M},{K}>", "scan8_exact"

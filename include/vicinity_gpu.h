@@ -321,6 +321,12 @@ int vgpu_test_polar_factor(const float *m, size_t d, float *r);
  * l2_distance_squared / 1 - dot (distance.rs:78-109). */
 int vgpu_test_bound_fast_tau(size_t d, size_t M, size_t ds, float qn, float cmax, float rmax,
                              float t0max, float *out);
+/* The scan by inverted list's score (bf16x3, padded_d dimensions) against
+ * the ADC distance, for |r|^2 = t0 and decoded residuals up to ymax. */
+int vgpu_test_bound_list(size_t padded_d, size_t M, size_t ds, float t0, float ymax, float *out);
+/* Which scan a batch search of nq queries takes now: 0 the mode's own, 1 the
+ * scan by inverted list (a test hook; no device call). */
+int vgpu_test_scan_route(vgpu_ivfpq *h, size_t nq, size_t k, size_t nprobe, size_t rerank_pool, int *out);
 int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float *out_bf16x3, float *out_fp32);
 int vgpu_test_bound_flat(size_t d, int metric, float qn, float xn, int ib, float *out);
 /* Device-allocation failure injection (a test hook with no reference

@@ -1,0 +1,150 @@
+"""GPU parity of the scan by inverted list (k_scan_list.hip), the route of
+large 8-bit batches: ids equal to the oracle's and float32 distances
+bit-identical over every padding of the score product (subvector widths 1, 2,
+3, 4, 5, 8, 12; dimensions that are not whole 32-dimension steps), lists of
+ragged length, empty ones and lists shorter than a 16-entry tile, k from 1
+to 200 and beyond the candidates, reranked, with OPQ, and with more equal
+distances than the survivor buffers hold (the exhaustive rescue).  Also, on
+the CPU, its error bound against float32 emulations of the kernel."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def _print_case(msg):
+    print(f"[case] {msg}", flush=True)
+
+
+def _route(ix, nq, k, nprobe, pool=0):
+    from vicinity_amd import _lib
+
+    out = ctypes.c_int(-1)
+    _lib.check(_lib.load().vgpu_test_scan_route(ix._h, nq, k, nprobe, pool, ctypes.byref(out)))
+    return out.value
+
+
+def _index(oracle, rng, n, d, L, M, K, rotation=None, x=None, together=None):
+    """(GPU index, oracle index) over mixture data; the lists are cut from a
+    random assignment with ragged sizes, one empty and one of three entries
+    (rows `together` share a list)."""
+    import vicinity_amd as v
+
+    if x is None:
+        c = rng.standard_normal((40, d)).astype(np.float32)
+        x = c[rng.integers(0, 40, n)] + 0.5 * rng.standard_normal((n, d)).astype(np.float32)
+    x = oracle.normalize_rows(x.astype(np.float32))
+    cent = oracle.normalize_rows(x[rng.choice(n, L, replace=False)].copy())
+    sizes = rng.integers(1, 9, L).astype(np.float64)
+    assign = rng.choice(L, n, p=sizes / sizes.sum())
+    assign[assign == 1] = 2  # list 1 is empty
+    assign[assign == 3] = 4
+    assign[:3] = 3
+    if together is not None:
+        assign[together] = 5
+    order = np.argsort(assign, kind="stable").astype(np.uint32)
+    off = np.concatenate([[0], np.cumsum(np.bincount(assign, minlength=L))]).astype(np.uint64)
+    res = x - cent[assign]
+    if rotation is not None:
+        res = res @ rotation.T
+    ds = d // M
+    books = np.stack([res[rng.choice(n, K, replace=False), m * ds:(m + 1) * ds] for m in range(M)])
+    books = np.ascontiguousarray(books.astype(np.float32))
+    codes = np.empty((n, M), np.uint8)
+    for m in range(M):
+        s = res[:, m * ds:(m + 1) * ds]
+        codes[:, m] = ((s * s).sum(1)[:, None] - 2 * s @ books[m].T + (books[m] ** 2).sum(1)).argmin(1)
+    ix = v.IVFPQIndex(d, num_clusters=L, num_codebooks=M, codebook_size=K, nprobe=4,
+                      use_opq=rotation is not None)
+    ix.load_artifacts(cent, books, off, order, codes, vectors=x, rotation=rotation)
+    oix = oracle.Index(cent, books.reshape(-1), off, order, codes, np.arange(n, dtype=np.uint32), x, M, K,
+                       rotation)
+    return ix, oix, x
+
+
+def _same(ix, oix, q, k, P, pool=0, route=1):
+    assert _route(ix, len(q), k, P, pool) == route, (len(q), k, P, pool)
+    ids, dists = ix.batch_search(q, k, nprobe=P, rerank_pool=pool or None)
+    oids, odists = oix.search_batch(q, k, P, rerank_pool=pool)
+    assert np.array_equal(ids, oids), (k, P, pool)
+    assert dists.tobytes() == odists.tobytes(), (k, P, pool)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,M,K", [(25, 25, 256), (50, 25, 256), (36, 12, 256), (100, 25, 256),
+                                   (60, 12, 64), (96, 12, 256), (72, 6, 256), (104, 13, 100)])
+def test_padded_shapes(oracle, d, M, K):
+    _print_case(f"list scan d={d} M={M} ksub={K}")
+    rng = np.random.default_rng(7 * d + M)
+    ix, oix, x = _index(oracle, rng, 6000, d, 24, M, K)
+    for nq, k, P in [(3001, 10, 9), (2999, 1, 12), (2500, 100, 24), (2500, 200, 7)]:
+        q = (x[rng.integers(0, len(x), nq)] + 0.2 * rng.standard_normal((nq, d))).astype(np.float32)
+        q = np.tile(q, (int(0.085e9 // (nq * P * 250 * M)) + 1, 1))  # enough work for the route
+        _same(ix, oix, q, k, P)
+    _same(ix, oix, q, 10, 9, pool=60)
+
+
+@pytest.mark.gpu
+def test_more_results_than_entries_and_rotated_residuals(oracle):
+    rng = np.random.default_rng(3)
+    _print_case("list scan: k beyond the probed entries")
+    ix, oix, x = _index(oracle, rng, 900, 100, 30, 25, 256)
+    q = x[rng.integers(0, 900, 70_000)] + 0.1 * rng.standard_normal((70_000, 100)).astype(np.float32)
+    _same(ix, oix, q[:60_000].astype(np.float32), 150, 2)
+    _print_case("list scan: OPQ")
+    rot = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((64, 64)))[0].astype(np.float32))
+    ix, oix, x = _index(oracle, rng, 5000, 64, 16, 16, 64, rotation=rot)
+    q = x[rng.integers(0, 5000, 1500)] + 0.2 * rng.standard_normal((1500, 64)).astype(np.float32)
+    for k, P in [(10, 5), (100, 16)]:
+        _same(ix, oix, q.astype(np.float32), k, P)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("copies,k", [(300, 10), (1500, 100), (9000, 10)])
+def test_equal_distances_beyond_the_buffers(oracle, copies, k):
+    """Copies of one vector: more entries within the bound than are rescored
+    (300, 1500) or kept (9000); ties come back in insertion order."""
+    _print_case(f"list scan: {copies} equal entries, k {k}")
+    rng = np.random.default_rng(copies)
+    x = rng.standard_normal((4000, 100)).astype(np.float32)
+    x = np.concatenate([np.repeat(x[:1], copies, axis=0), x])
+    perm = rng.permutation(len(x))
+    ix, oix, xn = _index(oracle, rng, len(x), 100, 16, 25, 256, x=x[perm], together=perm < copies)
+    q = np.concatenate([np.repeat(x[:1], 40, axis=0), x[rng.integers(0, len(x), 2000)]])
+    q = (q + 1e-3 * rng.standard_normal(q.shape)).astype(np.float32)
+    _same(ix, oix, q, k, 16)
+    assert ix.last_stats()["fallback_queries"] >= 40
+
+
+@pytest.mark.parametrize("d,M,scale", [(32, 8, 1.0), (96, 48, 0.05), (128, 16, 30.0)])
+def test_error_bound(oracle, d, M, scale):
+    """|a - e| <= list_tau with a from bf16x3 products in float32 (started
+    from -|y|^2 / 2, summed in order or truncated) and e the reference's
+    float32 distance; without its product term the bound fails."""
+    from test_proof_bounds import bf16_split, seq_sum
+
+    from vicinity_amd import _lib
+
+    rng = np.random.default_rng(d)
+    F32 = np.float32
+    r = (scale * rng.standard_normal((200, d))).astype(F32)
+    y = (r + scale * 10.0 ** rng.uniform(-3, 0, (200, 1)) * rng.standard_normal((200, d))).astype(F32)
+    yn = np.sum(y.astype(np.float64) ** 2, 1)
+    rh, rl = bf16_split(r)
+    yh, yl = bf16_split(y)
+    terms = np.concatenate([(-0.5 * yn).astype(F32)[:, None], yh * rl, yl * rh, yh * rh], 1).astype(F32)
+    t0 = seq_sum((r * r).astype(F32))
+    diff = (r - y).astype(F32)
+    e = seq_sum(seq_sum((diff * diff).astype(F32).reshape(200, M, -1)))
+    out = ctypes.c_float()
+    worst = 0.0
+    for i in range(200):
+        D = seq_sum(terms[i:i + 1])[0]
+        a = F32(np.float64(t0[i]) - 2.0 * np.float64(D))
+        _lib.check(_lib.load().vgpu_test_bound_list(d, M, d // M, float(t0[i]), float(np.sqrt(yn[i])),
+                                                    ctypes.byref(out)))
+        err = abs(float(a) - float(e[i]))
+        assert err <= out.value, (i, err, out.value)
+        worst = max(worst, err / out.value)
+    assert worst > 1e-3  # the inputs come within reach of the bound

@@ -150,6 +150,8 @@ SIGNATURES = {
     "vgpu_test_polar_factor": (_i, [_vp, _sz, _vp]),
     "vgpu_test_set_rres_limit": (_i, [_H, _sz]),
     "vgpu_test_fail_device_allocations": (_i, [_sz, _sz]),
+    "vgpu_test_bound_list": (_i, [_sz, _sz, _sz, _f, _f, _vp]),
+    "vgpu_test_scan_route": (_i, [_vp, _sz, _sz, _sz, _sz, _vp]),
     "vgpu_test_bound_fast_tau": (_i, [_sz, _sz, _sz, _f, _f, _f, _f, _vp]),
     "vgpu_test_bound_coarse": (_i, [_sz, _f, _f, _vp, _vp]),
     "vgpu_test_bound_flat": (_i, [_sz, _ci, _f, _f, _ci, _vp]),

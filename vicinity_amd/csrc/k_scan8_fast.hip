@@ -1830,6 +1830,13 @@ static size_t static_lut_bytes(const DevIndex& ix) {
     }
 }
 
+// The codebook counts and subvector widths launch_scan8_fast fixes at compile time.
+bool scan8_fast_compiled(int M, int K, int ds) {
+    if (K != 256) return false;
+    const bool m = M == 4 || M == 8 || M == 16 || M == 32 || M == 48 || M == 64;
+    return m && (ds == 2 || ds == 3 || ds == 4 || ds == 6 || ds == 8 || ds == 12 || ds == 16);
+}
+
 size_t scan8_fast_lds_bytes(const DevIndex& ix, const ScanArgs& a) {
     size_t off[12];
     const size_t st = static_lut_bytes(ix);

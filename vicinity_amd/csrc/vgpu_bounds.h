@@ -47,6 +47,22 @@ __host__ __device__ inline float fast_tau(int d, int M, int ds, float qn, float 
     return 4.0f * (float)(d + M + ds + 8) * u * S + 1e-30f;
 }
 
+// Bound on |a - e| for the scan by inverted list: a = t0 - 2 D with
+// t0 = fl(|r|^2) and D = r.y - |y|^2 / 2 in bf16x3 MFMA products over dp padded
+// dimensions started from fl(-|y|^2 / 2), e the reference's distance of the
+// residual r to the codewords y, ||y|| <= ymax (u = 2^-24).  The dropped
+// product terms are within 3.01 * 2^-16 sum|r_j y_j|, the accumulation of 3 dp
+// products within 3 dp 2u (sum|r_j y_j| + |y|^2 / 2) (accumulation that
+// truncates), the start value within u |y|^2 / 2, t0 within (dp + 2) u |r|^2,
+// the last rounding within u (|r| + |y|)^2, and the reference's differences,
+// squares and sums within (ds + M + 3) u (|r| + |y|)^2; a quarter to spare.
+__host__ __device__ inline float list_tau(int dp, int M, int ds, float t0, float ymax) {
+    const float u = 5.9604645e-08f;
+    const float rn = sqrtf(t0) * 1.0001f, ry = rn * ymax, yy = ymax * ymax, rr = (rn + ymax) * (rn + ymax);
+    const float dot = (3.01f * 1.5258789e-05f + 7.0f * (float)dp * u) * ry + (3.5f * (float)dp + 1.0f) * u * yy;
+    return 1.25f * (2.0f * dot + ((float)dp + 4.0f) * u * t0 + (float)(ds + M + 6) * u * rr) + 1e-30f;
+}
+
 // Bound on |ranking key + ||q||^2 (metric 0) - exact distance| with the
 // exact distance l2_distance_squared / 1 - seq_dot in float32
 // (u = 2^-24, |q| <= qn, |x| <= xn): the bf16x3 product is within

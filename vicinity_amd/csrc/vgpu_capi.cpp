@@ -628,6 +628,22 @@ int vgpu_test_bound_fast_tau(size_t d, size_t M, size_t ds, float qn, float cmax
     });
 }
 
+int vgpu_test_bound_list(size_t padded_d, size_t M, size_t ds, float t0, float ymax, float* out) {
+    return guard([&] {
+        need(out && padded_d && M && ds, VGPU_ERR_INVALID_PARAMETER, "bad argument");
+        *out = vgpu::list_tau((int)padded_d, (int)M, (int)ds, t0, ymax);
+    });
+}
+
+int vgpu_test_scan_route(vgpu_ivfpq* h, size_t nq, size_t k, size_t nprobe, size_t rerank_pool, int* out) {
+    return guard([&] {
+        need(h && out, VGPU_ERR_INVALID_PARAMETER, "null argument");
+        std::shared_lock<std::shared_mutex> lk(h->ix->mu);
+        need(h->ix->built, VGPU_ERR_NOT_BUILT, "IVF-PQ index: search before build");
+        *out = h->ix->plan_search(nq, k, nprobe, rerank_pool, true).list ? 1 : 0;
+    });
+}
+
 int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float* out_bf16x3, float* out_fp32) {
     return guard([&] {
         need(out_bf16x3 && out_fp32 && d, VGPU_ERR_INVALID_PARAMETER, "bad argument");

@@ -595,8 +595,93 @@ void IvfpqIndex::upload_index() {
             d_tblk_off.release();
         }
     }
+    upload_list_scan();
     VGPU_HIP(hipGetLastError());
     VGPU_HIP(hipStreamSynchronize(stream));
+}
+
+// Round to nearest even bfloat16 bits of a finite float.
+static uint32_t host_bf16(float x) {
+    uint32_t u;
+    std::memcpy(&u, &x, 4);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+
+// Tiles, codeword table and dimension map of the scan by inverted list
+// (k_scan_list.hip).  Codewords or centroids that are not finite, or so large
+// that squared norms could overflow, leave the index without it.
+void IvfpqIndex::upload_list_scan() {
+    lshape = list_shape((int)d, (int)M, (int)K, (int)ds);
+    max_list = 0;
+    for (size_t l = 0; l < L; l++) max_list = std::max<uint32_t>(max_list, (uint32_t)(offsets[l + 1] - offsets[l]));
+    // the score kernel's buffer loads take 32-bit byte offsets
+    uint64_t tiles = 0;
+    for (size_t l = 0; l < L; l++) tiles += (offsets[l + 1] - offsets[l] + 15) / 16;
+    if (tiles * 256 * lshape.LW >= ((uint64_t)1 << 32) - 256) lshape.ok = false;
+    if (!(dix.cmax < 1e15f) || !(dix.rmax < 1e15f)) lshape.ok = false;
+    for (float x : centroids) lshape.ok = lshape.ok && std::isfinite(x);
+    for (float x : codebooks) lshape.ok = lshape.ok && std::isfinite(x);
+    if (!lshape.ok) {
+        d_lcodes.release();
+        d_ltable.release();
+        d_ltoff.release();
+        d_lbias.release();
+        d_lcent.release();
+        d_dimmap.release();
+        return;
+    }
+    const int dsp = lshape.dsp, parts = lshape.parts, Mt = lshape.KT * 32 / dsp;
+    std::vector<uint32_t> toff(L + 1, 0), table(lshape.table_bytes / 4, 0u);
+    for (size_t l = 0; l < L; l++) toff[l + 1] = toff[l] + (uint32_t)((offsets[l + 1] - offsets[l] + 15) / 16);
+    std::vector<int> map((size_t)lshape.KT * 32, -1);
+    for (int mv = 0; mv < Mt; mv++)
+        for (int o = 0; o < dsp; o++) {
+            const int m = mv / parts, j = mv % parts * dsp + o;  // dimension j of codebook m
+            if (mv >= lshape.Mv || j >= (int)ds) continue;
+            map[(size_t)mv * dsp + o] = m * (int)ds + j;
+            for (size_t k = 0; k < K; k++) {
+                const float x = codebooks[((size_t)m * K + k) * ds + j];
+                const uint32_t hi = host_bf16(x);
+                float hf;
+                const uint32_t hb = hi << 16;
+                std::memcpy(&hf, &hb, 4);
+                const uint32_t lo = host_bf16(x - hf);
+                // a codeword: dsp high halves, then dsp low halves; for 8 the
+                // low halves are a second table
+                uint16_t* cw = reinterpret_cast<uint16_t*>(table.data());
+                const size_t c = (size_t)mv * K + k;
+                cw[dsp == 8 ? c * 8 + o : c * 2 * dsp + o] = (uint16_t)hi;
+                cw[dsp == 8 ? table.size() + c * 8 + o : c * 2 * dsp + dsp + o] = (uint16_t)lo;
+            }
+        }
+    std::vector<double> cwn(M * K, 0.0);
+    for (size_t i = 0; i < M * K; i++)
+        for (size_t j = 0; j < ds; j++) cwn[i] += (double)codebooks[i * ds + j] * codebooks[i * ds + j];
+    DevBuf<double> d_cwn;
+    d_cwn.upload(cwn.data(), cwn.size(), stream);
+    d_ltoff.upload(toff.data(), L + 1, stream);
+    d_ltable.upload(table.data(), table.size(), stream);
+    d_dimmap.upload(map.data(), map.size(), stream);
+    std::vector<float> pc;  // centroids in padded order
+    if (!lshape.contig) {
+        const size_t ld = map.size();
+        pc.assign(L * ld, 0.0f);
+        for (size_t l = 0; l < L; l++)
+            for (size_t j = 0; j < ld; j++)
+                if (map[j] >= 0) pc[l * ld + j] = centroids[l * d + map[j]];
+        d_lcent.upload(pc.data(), pc.size(), stream);
+    } else {
+        d_lcent.release();
+    }
+    d_lcodes.reserve((size_t)toff[L] * 64 * lshape.LW);
+    d_lbias.reserve((size_t)toff[L] * 16);
+    dix.ltoff = d_ltoff.p;
+    dix.ltiles = toff[L];
+    dix.ltable = d_ltable.p;
+    dix.lcodes = d_lcodes.p;
+    dix.lbias = d_lbias.p;
+    launch_list_tiles(dix, d_cwn.p, lshape, d_lcodes.p, d_lbias.p, stream);
+    VGPU_HIP(hipStreamSynchronize(stream));  // before d_cwn and the host arrays go
 }
 
 static int fast_keep(size_t kout) {
@@ -664,7 +749,43 @@ vgpu_search_stats IvfpqIndex::last_stats() {
     return stats;
 }
 
-SearchPlan IvfpqIndex::plan_search(size_t nq, size_t k, size_t nprobe, size_t pool) const {
+// Whether a search of nq queries takes the scan by inverted list, and its
+// buffer sizes.  Its fixed cost is about 40 us of launches above the FAST
+// scan's; per million scanned entries it costs 0.7 us (25 dimensions) to 1.6
+// us (128), where the FAST scan's lookups cost about 2.2 us at 8 codebooks, 3
+// at 16 and 9 at 48 (15 to 20 where the codebook count or the subvector width is
+// not one it is compiled for, and the EXACT scan of an OPQ index 22), and a
+// large k narrows the gap (its rescoring is the same).  Measured, FAST -> by
+// list: 1M x 128, M 16, k 10, 15M entries 149 -> 151 us, 39M 225 -> 180; k 100,
+// 39M 303 -> 314, 68M 461 -> 454; 300k x 32, M 8, 19M 113 -> 121, 76M 235 ->
+// 170; 1M x 96, M 48, 8M 166 -> 147; 1M x 100, M 25, 4M 203 -> 136; OPQ 500k x
+// 128, 0.8M 166 -> 154, 8M 309 -> 202.  A few wide codebooks cost few lookups
+// and many products: 300k x 96, M 8, 38M 208 -> 285.
+static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
+    if (!ix.lshape.ok || ix.mode != VGPU_MODE_FAST || pl.wide || pl.P == 0 || pl.kout > 256 || ix.L > SL_MAX_LISTS ||
+        (pl.opq && !ix.lshape.contig))
+        return false;
+    int sb = 0;
+    while (((size_t)1 << sb) < pl.P) sb++;
+    pl.tbits = std::min(26, 32 - sb);
+    if (ix.max_list >= (1u << pl.tbits)) return false;
+    const double pairs = (double)nq * pl.P, lookups = pairs * ix.n() / ix.L * ix.M;
+    if (pairs < 1.5 * ix.L) return false;
+    if (pl.opq) {
+        if (lookups < 0.02e9) return false;
+    } else if (!scan8_fast_compiled((int)ix.M, (int)ix.K, (int)ix.ds)) {
+        if (lookups < 0.08e9) return false;
+    } else if (lookups < 0.35e9 + 0.005e9 * (double)pl.kout || 10 * ix.M < (size_t)ix.lshape.KT * 32) {
+        return false;
+    }
+    pl.tcap = pl.kout <= 128 ? 32 : 64;
+    pl.cap = 4096;
+    pl.rcap = 256;
+    while ((size_t)pl.rcap < 4 * pl.kout) pl.rcap <<= 1;
+    return true;
+}
+
+SearchPlan IvfpqIndex::plan_search(size_t nq, size_t k, size_t nprobe, size_t pool, bool by_list) const {
     SearchPlan pl;
     if (pool && !has_vectors)
         throw Error(VGPU_ERR_UNSUPPORTED, "search_reranked after compact(): raw vectors were dropped");
@@ -674,6 +795,7 @@ SearchPlan IvfpqIndex::plan_search(size_t nq, size_t k, size_t nprobe, size_t po
     pl.kout = pool ? std::max(pool, k) : k;  // search.rs:1144
     if (pool && pl.kout > RERANK_MAX)
         throw Error(VGPU_ERR_UNSUPPORTED, "rerank_pool above " + std::to_string(RERANK_MAX) + " is not supported");
+    pl.opq = !rotation.empty();
     pl.wide = pl.P > 1024 || pl.kout > 2048;
     if (pl.P > SEL_WIDE_MAX)  // min(nprobe, nlist) lists sorted in LDS
         throw Error(VGPU_ERR_UNSUPPORTED, "probing more than " + std::to_string(SEL_WIDE_MAX) +
@@ -700,13 +822,16 @@ SearchPlan IvfpqIndex::plan_search(size_t nq, size_t k, size_t nprobe, size_t po
                                                   std::to_string(lds) +
                                                   " bytes, above the 160 KiB of LDS per workgroup");
     }
-    pl.opq = !rotation.empty();
     pl.fused = coarse_fused_supported((int)d, (int)pl.P);
-    pl.t2 = pl.P && K != 16 && mode == VGPU_MODE_FAST && !pl.opq && !pl.wide && scan8_fast_uses_tables(dix);
+    pl.list = by_list && use_list_scan(*this, nq, pl);
+    pl.t2 = pl.P && K != 16 && mode == VGPU_MODE_FAST && !pl.opq && !pl.wide && !pl.list && scan8_fast_uses_tables(dix);
     size_t chunk = std::max<size_t>(1, std::min<size_t>(nq, ((size_t)1 << 28) / std::max<size_t>(L, 1)));
     chunk = std::min<size_t>(chunk, 65536);
     if (pl.t2)  // tables of a chunk within 256 MiB
         chunk = std::max<size_t>(1, std::min<size_t>(chunk, ((size_t)1 << 26) / ((size_t)M * K)));
+    if (pl.list)  // survivors of a chunk within 512 MiB, its pairs within 2^22
+        chunk = std::max<size_t>(1, std::min({chunk, ((size_t)1 << 29) / ((size_t)pl.cap * 8), ((size_t)1 << 22) / pl.P,
+                                              ((size_t)1 << 29) / d}));
     if (pl.opq && pl.P)
         chunk = std::max<size_t>(1, std::min<size_t>(chunk, ((size_t)1 << 28) / (pl.P * d)));
     pl.chunk = chunk;
@@ -744,6 +869,37 @@ size_t IvfpqIndex::ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) c
     carve(w.flag_list, c);
     if (pl.opq) carve(w.rres, c * pl.P * d);
     if (pl.t2) carve(w.t2, c * M * K);
+    if (pl.list) {
+        ListWs& lw = w.list;
+        const size_t np = c * pl.P, ni = list_max_items(c, pl.P, L);
+        lw.sh = lshape;
+        lw.tcap = pl.tcap;
+        lw.cap = pl.cap;
+        lw.rcap = pl.rcap;
+        lw.tbits = pl.tbits;
+        lw.dimmap = d_dimmap.p;
+        carve(lw.cnt, (size_t)SL_COUNT_WG * L);
+        carve(lw.first, (size_t)SL_COUNT_WG * L);
+        carve(lw.first1, (size_t)SL_COUNT_WG * L);
+        carve(lw.heads, 4 + SL_RESCUE);
+        lw.rescued = lw.heads + 4;
+        carve(lw.rescue, SL_RESCUE * pl.kout);
+        lw.ld = lshape.contig ? (int)d : lshape.KT * 32;
+        lw.cent = lshape.contig ? d_centroids.p : d_lcent.p;
+        if (!lshape.contig) carve(lw.padded, c * (size_t)lw.ld);
+        carve(lw.pos, np);
+        carve(lw.tbase, np);
+        carve(lw.pairs, np);
+        carve(lw.pairs1, np);
+        carve(lw.items, ni);
+        carve(lw.items1, ni);
+        carve(lw.t0, np);
+        carve(lw.scount, c);
+        carve(lw.ntiles, c);
+        carve(lw.bound, c);
+        carve(lw.gbound, c * 16 * pl.tcap);
+        carve(lw.surv, c * pl.cap);
+    }
     if (out) *out = w;
     return (off + 255) & ~(size_t)255;
 }
@@ -861,7 +1017,7 @@ void IvfpqIndex::run_search(const float* d_q, size_t nq, const SearchPlan& pl, c
         if (allp) VGPU_HIP(hipEventRecord(ev[3], s));
         // scan-only timing: the FAST kernel's dispatch records the two events
         // itself; the other scan kernels are bracketed by marker events
-        const bool scan_fast = K != 16 && mode == VGPU_MODE_FAST && !pl.opq && !pl.wide;
+        const bool scan_fast = K != 16 && mode == VGPU_MODE_FAST && !pl.opq && !pl.wide && !pl.list;
         if (scanp && !scan_fast) VGPU_HIP(hipEventRecord(ws->sev[4 * ci], s));
         ScanArgs a;
         a.qn = w.qn;
@@ -884,6 +1040,11 @@ void IvfpqIndex::run_search(const float* d_q, size_t nq, const SearchPlan& pl, c
         if (K == 16) {
             a.kk = (int)kout;
             launch_fastscan(dix, a, s);
+            if (allp) VGPU_HIP(hipEventRecord(ev[4], s));
+            if (scanp) VGPU_HIP(hipEventRecord(ws->sev[4 * ci + 1], s));
+        } else if (pl.list) {
+            a.kk = (int)kout;
+            launch_scan_list(dix, a, w.list, s);
             if (allp) VGPU_HIP(hipEventRecord(ev[4], s));
             if (scanp) VGPU_HIP(hipEventRecord(ws->sev[4 * ci + 1], s));
         } else if (scan_fast) {
@@ -988,7 +1149,7 @@ void IvfpqIndex::search_device(const float* d_q, size_t nq, size_t k, size_t npr
         stats = st;
         return;
     }
-    const SearchPlan pl = plan_search(nq, k, nprobe, pool);
+    const SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
     WsLease ws(*this, take_ws());
     if (!s) s = ws->stream;
     ws.used = s;
@@ -1073,7 +1234,8 @@ vgpu_memory_report IvfpqIndex::memory_usage() {
     size_t dev = d_centroids.bytes() + d_codebooks.bytes() + d_bias.bytes() + d_vectors.bytes() +
                  d_rotation.bytes() + d_cb16.bytes() + d_offsets.bytes() + d_list_ids.bytes() +
                  d_doc_ids.bytes() + d_pack_off.bytes() + d_codes.bytes() + d_packed.bytes() +
-                 d_tblocks.bytes() + d_tblk_off.bytes() + d_ecat.bytes() + b_cb16.bytes() + b_dots.bytes() +
+                 d_tblocks.bytes() + d_tblk_off.bytes() + d_lcodes.bytes() + d_ltable.bytes() + d_ltoff.bytes() +
+                 d_lbias.bytes() + d_lcent.bytes() + d_dimmap.bytes() + d_ecat.bytes() + b_cb16.bytes() + b_dots.bytes() +
                  b_cflag_list.bytes() + b_cflag_count.bytes() +
                  b_overflow.bytes();
     {
@@ -1093,7 +1255,7 @@ void IvfpqIndex::search_host(const float* q, size_t nq, size_t k, size_t nprobe,
         if (!std::isfinite(q[i])) throw Error(VGPU_ERR_INVALID_PARAMETER, "query contains a non-finite value");
     if (!built) throw Error(VGPU_ERR_NOT_BUILT, "IVF-PQ index: search before build");
     if (nq == 0 || k == 0) return;
-    const SearchPlan pl = plan_search(nq, k, nprobe, pool);
+    const SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
     WsLease ws(*this, take_ws());
     hipStream_t s = ws->stream;
     ws->q.upload(q, nq * d, s);

@@ -38,6 +38,15 @@ struct DevIndex {
     const float* tbias = nullptr;
     const uint32_t* tblk_off = nullptr;// [L+1]
     uint32_t tblk_count = 0;           // blocks (one of slack past the last list's)
+    // The scan by inverted list (k_scan_list.hip; null when the shape is not
+    // supported): 16-entry tiles of every list, tiles ltoff[l] .. ltoff[l + 1]
+    // of list l, as code bytes in the order the matrix-core lanes read them
+    // and -|y|^2 / 2 per entry, and the bf16 hi/lo codewords.
+    const uint32_t* lcodes = nullptr;
+    const float* lbias = nullptr;
+    const uint32_t* ltable = nullptr;
+    const uint32_t* ltoff = nullptr;   // [L+1]
+    uint32_t ltiles = 0;
     float cmax = 0.f;                  // max ||c||
     float rmax = 0.f;                  // max ||decoded residual||
 };
@@ -160,6 +169,67 @@ size_t scan8_fast_lds_bytes(const DevIndex& ix, const ScanArgs& a);
 void launch_scan8_fast(const DevIndex& ix, const ScanArgs& a, hipStream_t s, hipEvent_t t0 = nullptr,
                        hipEvent_t t1 = nullptr);
 
+// ---- scan by inverted list (k_scan_list.hip) ----
+// Shape of its score product (list_shape).
+struct ListShape {
+    int dsp = 0;    // padded dimensions per (virtual) codebook: 1, 2, 4 or 8
+    int parts = 0;  // virtual codebooks per codebook
+    int Mv = 0;     // virtual codebooks
+    int KT = 0;     // 32-dimension steps
+    int LW = 0;     // code words per lane and tile
+    bool contig = false;  // padded dimension j is dimension j, rows of whole float4s
+    bool ok = false;
+    size_t table_bytes = 0;
+};
+ListShape list_shape(int d, int M, int K, int ds);
+#define SL_SLOT_BITS 10   // probe slots of a pair word (the rest: query of the chunk)
+#define SL_TCAP_MAX 160   // sample tiles per query, at most
+// Queries each workgroup of the pair count takes: at most 96 workgroups, whose
+// counts of every list are kept apart.
+#define SL_COUNT_WG 96
+inline int list_count_queries(int nq) {
+    const int q = (nq + SL_COUNT_WG - 1) / SL_COUNT_WG;
+    return q < 16 ? 16 : q;
+}
+#define SL_RESCUE 512       // workgroups of the flagged queries' exhaustive scan
+#define SL_MAX_LISTS 32768  // the pair count's LDS
+// Device workspace of one chunk (sizes in ws_layout).
+struct ListWs {
+    ListShape sh;
+    int tcap = 0;   // sample tiles per query
+    int cap = 0;    // survivors per query
+    int rcap = 0;   // rescored survivors per query
+    int tbits = 0;  // entry bits of a survivor's label (slot << tbits | entry)
+    int qw = 0, nwg = 0;  // queries per counting workgroup, counting workgroups
+    const int* dimmap = nullptr;  // [32 KT] dimension of each padded dimension, -1: padding
+    // rows of the score product, ld floats each: the normalised queries and
+    // the centroids, or (not contig) copies in padded order
+    int ld = 0;
+    const float *rows = nullptr, *cent = nullptr;
+    float* padded = nullptr;      // [nq ld] the queries' padded copy, filled by the pair count
+    uint32_t* cnt = nullptr;      // [nwg L] pairs (low half) and sample pairs (high half) of each list
+    uint32_t *first = nullptr, *first1 = nullptr;  // [nwg L] first pair, first sample pair
+    uint32_t* heads = nullptr;    // [4] sample pairs, sample items, pairs, items; zeroed with rescued
+    uint32_t* pos = nullptr;      // [nq P] place in the (workgroup, list)'s pairs, in its sample pairs
+    uint32_t* tbase = nullptr;    // [nq P] sample tiles of the query's nearer lists
+    uint32_t *pairs = nullptr, *pairs1 = nullptr;  // [nq P] pair words by list
+    uint4 *items = nullptr, *items1 = nullptr;
+    float* t0 = nullptr;          // [nq P] |r|^2
+    uint32_t *scount = nullptr, *ntiles = nullptr;  // [nq] survivors, sample tiles
+    float* bound = nullptr;       // [nq]
+    float* gbound = nullptr;      // [nq 16 tcap] upper bounds of the sample's distances
+    uint2* surv = nullptr;        // [nq cap] (label, distance bits)
+    uint32_t* rescued = nullptr;  // [SL_RESCUE] finished workgroups of each flagged query
+    uint64_t* rescue = nullptr;   // [SL_RESCUE kout] their keys
+};
+// Work items of a chunk of nq queries, at most: blocks of 64 pairs x 16 segments.
+inline size_t list_max_items(size_t nq, size_t P, size_t L) { return 16 * (nq * P / 64 + (L < nq * P ? L : nq * P)); }
+// lcodes / lbias of every list (cwn: |codeword|^2 in float64).
+void launch_list_tiles(const DevIndex& ix, const double* cwn, const ListShape& sh, uint32_t* lcodes, float* lbias,
+                       hipStream_t s);
+// The whole scan of a chunk: rows written like launch_scan8_fast's; queries
+// whose survivors do not fit are appended to a.flag_list and scanned exhaustively.
+void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& w, hipStream_t s);
 #define QSTAT_WORDS 4
 // Search statistics: entries scanned, fallbacks, flushes, appends, fallbacks
 // from ties, second passes; counter i lives at counters[i * COUNTER_STRIDE]
@@ -226,6 +296,8 @@ void launch_bias(const DevIndex& ix, float* bias, hipStream_t s);
 #define TBLK_BYTES(M) (16 * (size_t)(M) + 64)
 // Whether the FAST scan reads transposed blocks for this shape.
 bool scan8_fast_blocks_supported(int M, int K, int ds);
+// Whether the FAST scan has this codebook count and width at compile time.
+bool scan8_fast_compiled(int M, int K, int ds);
 // The FAST scan shapes whose per-query tables come from launch_t2_tables
 // (16 codebooks of 256 codewords on transposed blocks, ds 2, 4 or 8).
 bool scan8_fast_uses_tables(const DevIndex& ix);

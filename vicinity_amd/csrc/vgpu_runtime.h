@@ -84,6 +84,10 @@ struct SearchPlan {
     // nprobe above 1024 or kout above 2048: probes chosen from exact scores of
     // every list, scans in EXACT (or FastScan) mode with per-slot list reads
     bool wide = false;
+    // the scan by inverted list (k_scan_list.hip), its sample tiles, survivor
+    // buffer and label bits
+    bool list = false;
+    int tcap = 0, cap = 0, rcap = 0, tbits = 0;
 };
 
 // Device pointers of one call's workspace, carved from one arena
@@ -97,6 +101,7 @@ struct WsPtrs {
     uint32_t* qbad = nullptr;  // per chunk query: 1 when the query holds a NaN or an infinity
     float* fdots = nullptr;  // coarse fallback: dot-product rows of the first flagged queries
     unsigned long long* scal = nullptr;  // per-call scalars (counters, flag-list lengths)
+    ListWs list;             // the scan by inverted list
 };
 
 // Per-call device scalars: counter i at word i * COUNTER_STRIDE, then the
@@ -166,6 +171,11 @@ struct IvfpqIndex {
     DevBuf<uint32_t> d_offsets, d_list_ids, d_doc_ids, d_pack_off;
     DevBuf<uint8_t> d_codes, d_packed, d_tblocks;
     DevBuf<uint32_t> d_tblk_off;
+    DevBuf<uint32_t> d_lcodes, d_ltable, d_ltoff;  // scan by inverted list
+    DevBuf<float> d_lbias, d_lcent;
+    DevBuf<int> d_dimmap;
+    ListShape lshape;
+    uint32_t max_list = 0;          // entries of the longest list
     DevIndex dix;
 
     // build workspace (k-means assignment), used under the exclusive lock
@@ -205,7 +215,8 @@ struct IvfpqIndex {
     // The rotation of an OPQ index built elsewhere (before load); null clears it.
     void set_rotation(const float* R);
     // The probe count, plan and shape checks of a search of nq queries.
-    SearchPlan plan_search(size_t nq, size_t k, size_t nprobe, size_t pool) const;
+    // by_list: whether the scan by inverted list may be chosen.
+    SearchPlan plan_search(size_t nq, size_t k, size_t nprobe, size_t pool, bool by_list = false) const;
     // Bytes of a plan's workspace arena; with a base, also the pointers into it.
     size_t ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) const;
     // Device-pointer batch search on stream s (null: the borrowed workspace's
@@ -269,6 +280,7 @@ struct IvfpqIndex {
     void rotate_slots(const float* d_qn, size_t nq, size_t P, const uint32_t* d_lists, float* out,
                       hipStream_t s);
     void snapshot_list_masks();
+    void upload_list_scan();  // the arrays of the scan by inverted list
     void refresh_categories(hipStream_t s);
 };
 
