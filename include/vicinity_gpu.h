@@ -328,6 +328,7 @@ int vgpu_test_bound_list(size_t padded_d, size_t M, size_t ds, float t0, float y
  * scan by inverted list (a test hook; no device call). */
 int vgpu_test_scan_route(vgpu_ivfpq *h, size_t nq, size_t k, size_t nprobe, size_t rerank_pool, int *out);
 int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float *out_bf16x3, float *out_fp32);
+/* ib -1: the flat score's bound before packing (k above 32). */
 int vgpu_test_bound_flat(size_t d, int metric, float qn, float xn, int ib, float *out);
 /* Device-allocation failure injection (a test hook with no reference
  * counterpart): after `after` more device allocations by the library succeed,

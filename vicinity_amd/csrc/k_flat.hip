@@ -14,7 +14,7 @@
 // and rescores it; a query that fails the check is searched exhaustively with
 // the exact arithmetic.
 //
-// flat_rank_kernel (d <= 128): bf16x3 MFMA products (q.x ~ qh.xh + qh.xl +
+// flat_rank_kernel (d <= 256): bf16x3 MFMA products (q.x ~ qh.xh + qh.xl +
 // ql.xh, as the coarse quantiser), 128 queries per workgroup held in
 // registers, the slice's vectors streamed through LDS two 16-vector tiles at
 // a time (pre-split into bf16 hi/lo, tile-major).  Each score is compared
@@ -181,12 +181,12 @@ __global__ __launch_bounds__(256) void flat_partial_kernel(
 }
 
 
-// ---- bf16x3 ranking kernel (d <= 128) ------------------------------------
+// ---- bf16x3 ranking kernel (d <= 256) ------------------------------------
 
 #define FR_TPS 2    // database tiles (16 vectors each) per pipeline stage
 #define FR_QBW 2    // query blocks (16 queries each) per wave
 #define FR_ROWS (4 * FR_QBW * 16)  // queries per workgroup
-#define FR_J 4      // keys each lane keeps per row (and sorts per lane at the end)
+#define FR_MAXD 256
 #define FR_BIG 3.0e38f
 
 // Round to nearest even bfloat16 bits (finite inputs); x = hi + lo + r with
@@ -196,26 +196,41 @@ __device__ __forceinline__ uint32_t fr_bf16_bits(float x) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-// Ascending list of the FR_J smallest keys: t_i' = med3(t_{i-1}, t_i, v) from
+// Keys each lane keeps per row: J.  The merge needs every list's J-th key above
+// its threshold, so J and the slices are chosen for few members per list: up to
+// k 32 a lane of one of 32 slices holds 0.06 of the k nearest and four keys
+// are enough; at k 100 it holds 0.2, with the keys within the error margin up
+// to twice that, and four keys would leave about 4% of the queries unproved,
+// six keys under 0.1%.
+#define FR_J_WIDE 6
+__host__ __device__ constexpr int fr_keys(int k) { return k <= 32 ? 4 : FR_J_WIDE; }
+
+// Ascending list of the J smallest keys: t_i' = med3(t_{i-1}, t_i, v) from
 // the bottom, t_0' = min(t_0, v).
-__device__ __forceinline__ void fr_insert(float (&t)[FR_J], float v) {
+template <int J>
+__device__ __forceinline__ void fr_insert(float (&t)[J], float v) {
 #pragma unroll
-    for (int i = FR_J - 1; i > 0; i--) t[i] = __builtin_amdgcn_fmed3f(t[i - 1], t[i], v);
+    for (int i = J - 1; i > 0; i--) t[i] = __builtin_amdgcn_fmed3f(t[i - 1], t[i], v);
     t[0] = fminf(t[0], v);
 }
 
+// Bounds: the matrix cores and, behind them, the J + 3 vector instructions per
+// score of the lists.  Whole search of 10,000 queries: 100k x 96, k 10
+// 0.72 ms; 250k x 128, k 100 2.12 ms, where fp32 products filtered into one
+// buffer per query took 68 ms.
+//
 // Workgroup (4 waves) = FR_ROWS queries x one database slice of tiles
 // [blockIdx.y * tps, ..) (tps <= 2^ib).  Wave w holds query blocks
 // FR_QBW w .. + FR_QBW - 1 (bf16 hi/lo A operands in registers); every stage
 // of FR_TPS tiles is copied to LDS once and multiplied by all of them.  The
 // lane of group g (lanes 16 g .. + 15) and column c scores rows 4 g .. + 3 of
 // each of its query blocks against vector 16 tile + c and keeps, per row, the
-// FR_J smallest keys (score with the low ib mantissa bits replaced by the
+// J smallest keys (score with the low ib mantissa bits replaced by the
 // tile's index in the slice).  At the end each row's 16 lanes write their
-// 16 FR_J keys as (fkey, vector index), unsorted (the merge selects), and a
-// bound every key the slice dropped is at or above: the FR_J-th key of every
+// 16 J keys as (fkey, vector index), unsorted (the merge selects), and a
+// bound every key the slice dropped is at or above: the J-th key of every
 // full lane list.
-template <int DT>
+template <int DT, int J>
 __global__ __launch_bounds__(256) void flat_rank_kernel(
     const float* __restrict__ Q, int nq, int d, const uint4* __restrict__ Xb_in,
     const float* __restrict__ Xnorm, int n, int metric, int kk, int tps, int ib, int splits,
@@ -261,13 +276,37 @@ __global__ __launch_bounds__(256) void flat_rank_kernel(
             al[qb][t] = u32x4{lb[0] | lb[1] << 16, lb[2] | lb[3] << 16, lb[4] | lb[5] << 16, lb[6] | lb[7] << 16};
         }
     }
-    float lst[FR_QBW][4][FR_J];
+    // Six keys: accumulators start from ||q||^2 (metric 0), so a score is the
+    // distance up to rounding and the keys near the threshold, which are small,
+    // lose only their own low bits to the tile index.  (With four keys the
+    // start values cost 2% and the margin is narrow enough without.)
+    floatx4 start[FR_QBW];
+#pragma unroll
+    for (int qb = 0; qb < FR_QBW; qb++) {
+        start[qb] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (J == 4 || metric != 0) continue;
+        float sq = 0.0f;  // row c's sum over the lane's dimensions
+        const float* qr = Q + (size_t)min(q0 + (FR_QBW * wave + qb) * 16 + c, nq - 1) * d;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int j = 32 * t + 8 * g + i;
+                const float x = j < d ? qr[j] : 0.0f;
+                sq = __builtin_fmaf(x, x, sq);
+            }
+        sq += __shfl_xor(sq, 16, 64);
+        sq += __shfl_xor(sq, 32, 64);
+#pragma unroll
+        for (int r = 0; r < 4; r++) start[qb][r] = __shfl(sq, 4 * g + r, 64);
+    }
+    float lst[FR_QBW][4][J];
 #pragma unroll
     for (int qb = 0; qb < FR_QBW; qb++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int j = 0; j < FR_J; j++) lst[qb][r][j] = FR_BIG;
+            for (int j = 0; j < J; j++) lst[qb][r][j] = FR_BIG;
 
     // Stage st: tiles tile0 + FR_TPS st .. + FR_TPS - 1 (chunks contiguous in
     // the packed copy, which is padded to whole groups of four tiles).
@@ -325,7 +364,7 @@ __global__ __launch_bounds__(256) void flat_rank_kernel(
         for (int i = 0; i < FR_TPS; i++) {
             xn[i] = snorm[(st & 1) * FR_TPS * 16 + i * 16 + c];
 #pragma unroll
-            for (int qb = 0; qb < FR_QBW; qb++) acc[i][qb] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int qb = 0; qb < FR_QBW; qb++) acc[i][qb] = start[qb];
         }
 #pragma unroll
         for (int t = 0; t < DT; t++) {
@@ -354,14 +393,14 @@ __global__ __launch_bounds__(256) void flat_rank_kernel(
     }
     if (nst > 0) epilogue(prev, prevn, nst - 1, true);
 
-    // Per row: every lane's FR_J keys as (fkey, vector index), ~0 past a
+    // Per row: every lane's J keys as (fkey, vector index), ~0 past a
     // short list, and the bound every dropped key is at or above: the
-    // FR_J-th key of every full lane list (all 16 FR_J keys are kept, kk =
-    // 16 FR_J, so no key of the lists themselves is dropped).
+    // J-th key of every full lane list (all 16 J keys are kept, kk =
+    // 16 J, so no key of the lists themselves is dropped).
 #pragma unroll
     for (int j = 0; j < 4 * FR_QBW; j++) {
         const int qb = j >> 2, r = j & 3;
-        const float tl = lst[qb][r][FR_J - 1];
+        const float tl = lst[qb][r][J - 1];
         uint32_t lb = tl < FR_BIG ? fkey(tl) : 0xffffffffu;
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) {
@@ -372,7 +411,7 @@ __global__ __launch_bounds__(256) void flat_rank_kernel(
         if (qrow < nq) {
             uint64_t* out = partial + ((size_t)qrow * splits + sl) * kk;
 #pragma unroll
-            for (int e = 0; e < FR_J; e++) {
+            for (int e = 0; e < J; e++) {
                 const float t = lst[qb][r][e];
                 const uint32_t col = (uint32_t)((tile0 + (int)(__float_as_uint(t) & ~kmask)) * 16 + c);
                 out[e * 16 + c] = t < FR_BIG ? ((uint64_t)fkey(t) << 32) | col : ~0ull;
@@ -561,15 +600,24 @@ __global__ __launch_bounds__(256) void flat_merge_kernel(
 // most FM_R) are compacted through LDS, rescored with the reference's
 // arithmetic and sorted in registers.  More than FM_R such keys, or no
 // proof: the query goes to the exhaustive fallback.
-#define FM_R 256
-template <int E>
+// With six keys the packing is bounded per key instead of over all scores: an
+// entry with score v (the key before packing) has |key - v| <= rel |key|,
+// rel = 2^(ib - 23), and |v - distance| <= tau up to the row's constant.  The k
+// smallest keys are <= A, so the k-th distance is within A + rel |A| + tau and
+// a member of the top k has a score <= V = A + rel |A| + 2 tau and a key <= V +
+// rel |V| (twice rel covers the rounding of these sums).
+// Above 32 keys or 128 dimensions nothing is proved for a query that is not
+// finite (or whose products could overflow): every vector is scored exactly
+// for it (threshold ~0).
+#define FM_MAX_NORM 1.0e15f
+template <int E, int FM_R>
 __global__ __launch_bounds__(256) void flat_merge_wave_kernel(
     const uint64_t* __restrict__ partial, const uint32_t* __restrict__ pbound, int splits, int kk,
     const float* __restrict__ Q, const float* __restrict__ Qsq, const float* __restrict__ X, int nq, int d,
     int k, int metric, float xmax, int ib, uint32_t* __restrict__ out_idx, float* __restrict__ out_dist,
     unsigned int* overflow, uint32_t* __restrict__ flag_list, uint32_t* __restrict__ fbv) {
     __shared__ uint64_t rbuf[4][FM_R];
-    __shared__ float qsh[4][128];  // d <= 128
+    __shared__ float qsh[4][FR_MAXD];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int q = blockIdx.x * 4 + wave;
     if (q >= nq) return;
@@ -590,6 +638,13 @@ __global__ __launch_bounds__(256) void flat_merge_wave_kernel(
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    if ((k > 32 || d > 128) && !(qsq < FM_MAX_NORM * FM_MAX_NORM)) {
+        if (lane == 0) {
+            fbv[q] = 0xffffffffu;
+            flag_list[atomicAdd(overflow, 1u)] = (uint32_t)q;
+        }
+        return;
+    }
     const int tot = splits * kk;
     uint64_t kv[E];
     const uint64_t* src = partial + (size_t)q * tot;
@@ -601,6 +656,16 @@ __global__ __launch_bounds__(256) void flat_merge_wave_kernel(
     int m = 0;  // valid keys (padding is ~0)
 #pragma unroll
     for (int e = 0; e < E; e++) m += (int)__popcll(__ballot(kv[e] != ~0ull));
+    uint32_t B = 0xffffffffu;
+    for (int sl = lane; sl < splits; sl += 64) {
+        const uint32_t b = pbound[(size_t)q * splits + sl];
+        B = b < B ? b : B;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t x = (uint32_t)__shfl_xor((int)B, o, 64);
+        B = x < B ? x : B;
+    }
     uint32_t fb = 0xffffffffu;  // keys whose high word is <= fb are rescored
     if (m >= k) {
         uint32_t T = 0;  // the (k-1)-th smallest high word: the largest v with < k words below it
@@ -611,29 +676,23 @@ __global__ __launch_bounds__(256) void flat_merge_wave_kernel(
             for (int e = 0; e < E; e++) below += (int)__popcll(__ballot((uint32_t)(kv[e] >> 32) < cand));
             if (below <= k - 1) T = cand;
         }
-        const float u = 5.9604645e-08f;
         const float qmax = sqrtf(qsq) * 1.0001f + 1e-30f;
-        const float tau = flat_bf16_tau(d, metric, qmax, xmax, ib);
-        fb = fkey(fkey_to_float(T) + 2.0f * tau);
+        if constexpr (FM_R > 256) {  // six keys
+            const float tau = flat_key_tau(d, metric, qmax, xmax), rel = exp2f((float)(ib - 22));
+            const float A = fkey_to_float(T), V = A + rel * fabsf(A) + 2.0f * tau;
+            fb = fkey(V + rel * fabsf(V));
+        } else {
+            fb = fkey(fkey_to_float(T) + 2.0f * flat_bf16_tau(d, metric, qmax, xmax, ib));
+        }
         fb = fb < 0xfffffffeu ? fb + 1u : 0xffffffffu;  // one ulp up: the bound is not rounded down
-        (void)u;
-        uint32_t B = 0xffffffffu;
-        for (int sl = lane; sl < splits; sl += 64) {
-            const uint32_t b = pbound[(size_t)q * splits + sl];
-            B = b < B ? b : B;
+    }
+    // fewer than k keys hold every vector when no list is full (B ~0)
+    if (m >= k ? !(B > fb) : B != 0xffffffffu) {
+        if (lane == 0) {
+            fbv[q] = fb;
+            flag_list[atomicAdd(overflow, 1u)] = (uint32_t)q;
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t x = (uint32_t)__shfl_xor((int)B, o, 64);
-            B = x < B ? x : B;
-        }
-        if (!(B > fb)) {
-            if (lane == 0) {
-                fbv[q] = fb;
-                flag_list[atomicAdd(overflow, 1u)] = (uint32_t)q;
-            }
-            return;
-        }
+        return;
     }
     // compact the keys <= fb into this wave's LDS row
     uint32_t cnt = 0;
@@ -669,14 +728,26 @@ __global__ __launch_bounds__(256) void flat_merge_wave_kernel(
         uint64_t r1[1] = {rescore((uint32_t)lane)};
         wave_sort_regs<1>(r1);
         emit(lane, r1[0]);
+        if (k > 64) emit(64 + lane, ~0ull);
         return;
     }
-    uint64_t r[FM_R / 64];
+    if constexpr (FM_R > 256) {
+        if (cnt > 256) {
+            uint64_t r[FM_R / 64];
 #pragma unroll
-    for (int e = 0; e < FM_R / 64; e++) r[e] = rescore((uint32_t)(e * 64 + lane));
-    wave_sort_regs<FM_R / 64>(r);
+            for (int e = 0; e < FM_R / 64; e++) r[e] = rescore((uint32_t)(e * 64 + lane));
+            wave_sort_regs<FM_R / 64>(r);
 #pragma unroll
-    for (int e = 0; e < FM_R / 64; e++) emit(e * 64 + lane, r[e]);
+            for (int e = 0; e < 2; e++) emit(e * 64 + lane, r[e]);  // k <= 112
+            return;
+        }
+    }
+    uint64_t r[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = rescore((uint32_t)(e * 64 + lane));
+    wave_sort_regs<4>(r);
+#pragma unroll
+    for (int e = 0; e < 2; e++) emit(e * 64 + lane, r[e]);
 }
 
 // Database slices per query block: enough blocks to fill the GPU, slices of
@@ -690,23 +761,27 @@ static int flat_splits(int nq, int n, int kk) {
     return sp;
 }
 
-// The bf16x3 ranking kernel serves d <= 128 and k <= 32; every slice keeps
-// all 16 FR_J keys of a row's lane lists, plus one bound word per (query,
-// slice) after the keys.
-static bool flat_rank_ok(int d, int k) { return d >= 1 && d <= 128 && k >= 1 && k <= 32; }
-static int flat_rank_keep(int k) {
-    (void)k;
-    return 16 * FR_J;
+// The bf16x3 ranking kernel serves d <= 256 and k <= 112 (every k that is
+// accepted); every slice keeps all 16 J keys of a row's lane lists, plus one
+// bound word per (query, slice) after the keys.
+// Rows above 128 dimensions or k above 32 take it only when every row is
+// finite and far from overflow; the rest keep the fp32 path.
+bool flat_rank_ok(int d, int k, bool plain_rows) {
+    return d >= 1 && d <= FR_MAXD && k >= 1 && k <= 112 && (plain_rows || (d <= 128 && k <= 32));
 }
+static int flat_rank_keep(int k) { return 16 * fr_keys(k); }
 
 // Slices for the ranking kernel: a whole number of stages (FR_TPS tiles)
-// each, enough workgroups for four waves of two per CU on 256 CUs, slices of
-// at least 64 tiles, and splits * kk merge entries within the merge buffer;
-// ib = the bits of a tile index within a slice.
+// each, and ib = the bits of a tile index within a slice.  Up to k 32: enough
+// workgroups for four waves of two per CU on 256 CUs, slices of at least 64
+// tiles.  Above: 32 slices whatever the batch, as long as a slice has three
+// tiles, so that few of the k nearest share a lane list.  At most 2048 (k 32)
+// or 3072 merge entries, which the merge holds in registers.
 static int flat_rank_splits(int nq, int n, int kk, int* tps, int* ib) {
     const int qb = (nq + FR_ROWS - 1) / FR_ROWS, ntiles = (n + 15) / 16;
+    const bool wide = kk == 16 * FR_J_WIDE;
     int sp = 1;
-    while (qb * sp < 2048 && 2 * sp * kk <= FL_BUF && ntiles / (2 * sp) >= 64) sp <<= 1;
+    while (sp < 32 && (wide || qb * sp < 2048) && ntiles / (2 * sp) >= (wide ? 3 : 64)) sp <<= 1;
     int t = (ntiles + sp - 1) / sp;
     t = (t + FR_TPS - 1) / FR_TPS * FR_TPS;  // whole stages: a stage never reaches past the padded copy
     int b = 1;
@@ -715,6 +790,9 @@ static int flat_rank_splits(int nq, int n, int kk, int* tps, int* ib) {
     *ib = b;
     return (ntiles + t - 1) / t;
 }
+
+// Queries of one pass above k 32: its kept keys stay within 1 GiB.
+int flat_rank_chunk() { return 40960; }
 
 // Exhaustive exact fallback of the unproved queries, spread over the GPU:
 // workgroup (s, i) finds the exact top-k of query flag_list[i] among vectors
@@ -736,11 +814,12 @@ __global__ __launch_bounds__(256) void flat_exact_slice_kernel(
 
 // nflag_dev (optional): the flagged-query count on the device; workgroups
 // past it (or past the grid) have nothing to do.
+template <int BUF>
 __global__ __launch_bounds__(256) void flat_exact_finish_kernel(
     const uint32_t* __restrict__ flag_list, int slices, int k, const uint64_t* __restrict__ in_keys,
     uint32_t* __restrict__ out_idx, float* __restrict__ out_dist, const unsigned int* nflag_dev) {
-    __shared__ uint64_t keys[FL_BUF];
-    __shared__ uint32_t pay[FL_BUF];
+    __shared__ uint64_t keys[BUF];
+    __shared__ uint32_t pay[BUF];
     const int i = blockIdx.x, tid = threadIdx.x;
     if (nflag_dev && (unsigned int)i >= *nflag_dev) return;
     const uint32_t q = flag_list[i];
@@ -758,12 +837,23 @@ __global__ __launch_bounds__(256) void flat_exact_finish_kernel(
     }
 }
 
+// slices * k keys per query: 2048 at most, or 32 x 112 on the ranking path.
+static void launch_exact_finish(int nf, const uint32_t* flag_list, int slices, int k, const uint64_t* keys,
+                                uint32_t* out_idx, float* out_dist, const unsigned int* nflag_dev, hipStream_t s) {
+    if (slices * k <= FL_BUF)
+        hipLaunchKernelGGL(flat_exact_finish_kernel<FL_BUF>, dim3(nf), dim3(256), 0, s, flag_list, slices, k, keys,
+                           out_idx, out_dist, nflag_dev);
+    else
+        hipLaunchKernelGGL(flat_exact_finish_kernel<2 * FL_BUF>, dim3(nf), dim3(256), 0, s, flag_list, slices, k,
+                           keys, out_idx, out_dist, nflag_dev);
+}
+
 // Fallback of the ranking path, workgroup (s, i) for query q = flag_list[i]
 // and ranking slice s (tiles s tps ..), fb = the query's rescoring threshold
-// fbv[q].  Lane c of a slice's row kept the FR_J smallest keys of vectors
+// fbv[q].  Lane c of a slice's row kept the J smallest keys of vectors
 // 16 (s tps + t) + c (t < tps) at partial[e 16 + c], sorted in e; a lane whose
-// list is not full dropped nothing, and one whose FR_J-th key exceeds fb
-// dropped no key <= fb.  The other lanes' columns are scanned with the exact
+// list is not full dropped nothing, and one whose J-th key exceeds fb
+// dropped no key <= fb (fb ~0: nothing is known, every lane counts).  The other lanes' columns are scanned with the exact
 // arithmetic, and the kept keys <= fb of the rest are rescored: every vector
 // with a key <= fb (the superset of the exact top-k the merge proved) is
 // scored exactly, so the slice's k smallest exact keys, written to out_keys
@@ -777,7 +867,7 @@ __global__ __launch_bounds__(256) void flat_rank_fallback_kernel(
     __shared__ uint64_t keys[FL_BUF];
     __shared__ uint32_t pay[FL_BUF];
     __shared__ uint32_t misc[12];
-    __shared__ float qs[128];  // d <= 128
+    __shared__ float qs[FR_MAXD];
     __shared__ uint32_t rescan[16];
     const int s = blockIdx.x, i = blockIdx.y, tid = threadIdx.x;
     const uint32_t q = flag_list[i];
@@ -787,24 +877,28 @@ __global__ __launch_bounds__(256) void flat_rank_fallback_kernel(
     for (int j = tid; j < d; j += blockDim.x) qs[j] = Q[(size_t)q * d + j];
     __syncthreads();
     if (pbound[(size_t)q * splits + s] > fb) {
-        if (tid >= 64) return;  // kk <= 64 kept keys: one wave
-        uint64_t r[1] = {~0ull};
-        if (tid < kk) {
-            const uint64_t key = src[tid];
+        if (tid >= 64) return;  // kk <= 128 kept keys: one wave
+        uint64_t r[2] = {~0ull, ~0ull};
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i2 = u * 64 + tid;
+            const uint64_t key = i2 < kk ? src[i2] : ~0ull;
             if (key != ~0ull && (uint32_t)(key >> 32) <= fb) {
                 const uint32_t idx = (uint32_t)key;
-                r[0] = cand_key(flat_exact(qs, X + (size_t)idx * d, d, metric), idx);
+                r[u] = cand_key(flat_exact(qs, X + (size_t)idx * d, d, metric), idx);
             }
         }
-        wave_sort_regs<1>(r);
-        if (tid < k) out[tid] = r[0];
+        wave_sort_regs<2>(r);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (u * 64 + tid < k) out[u * 64 + tid] = r[u];
         return;
     }
-    // the lanes to rescan: full list (FR_J-th key present) with that key <= fb
+    // the lanes to rescan: full list (J-th key present) with that key <= fb
     uint32_t nres = 0, resmask = 0;
     for (int c = 0; c < 16; c++) {
-        const uint64_t last = src[(FR_J - 1) * 16 + c];
-        if (last != ~0ull && (uint32_t)(last >> 32) <= fb) {
+        const uint64_t last = src[kk - 16 + c];
+        if (fb == 0xffffffffu || (last != ~0ull && (uint32_t)(last >> 32) <= fb)) {
             if (tid == 0) rescan[nres] = (uint32_t)c;
             nres++;
             resmask |= 1u << c;
@@ -844,8 +938,8 @@ void launch_flat_rank_fallback(const uint32_t* flag_list, int nflag, const uint3
         const int nf = nflag - f0 < 65535 ? nflag - f0 : 65535;
         hipLaunchKernelGGL(flat_rank_fallback_kernel, dim3(sp, nf), dim3(256), 0, s, flag_list + f0, fbv, partial,
                            pbound, sp, kk, tps, Q, X, n, d, k, metric, keys + (size_t)f0 * sp * k, nullptr);
-        hipLaunchKernelGGL(flat_exact_finish_kernel, dim3(nf), dim3(256), 0, s, flag_list + f0, sp, k,
-                           keys + (size_t)f0 * sp * k, out_idx, out_dist, nullptr);
+        launch_exact_finish(nf, flag_list + f0, sp, k, keys + (size_t)f0 * sp * k, out_idx, out_dist,
+                            nullptr, s);
     }
 }
 
@@ -859,12 +953,11 @@ void launch_flat_rank_fallback_dev(const uint32_t* flag_list, const unsigned int
     const uint32_t* pbound = reinterpret_cast<const uint32_t*>(partial + (size_t)nq * sp * kk);
     hipLaunchKernelGGL(flat_rank_fallback_kernel, dim3(sp, cap), dim3(256), 0, s, flag_list, fbv, partial, pbound,
                        sp, kk, tps, Q, X, n, d, k, metric, keys, nflag_dev);
-    hipLaunchKernelGGL(flat_exact_finish_kernel, dim3(cap), dim3(256), 0, s, flag_list, sp, k, keys, out_idx,
-                       out_dist, nflag_dev);
+    launch_exact_finish(cap, flag_list, sp, k, keys, out_idx, out_dist,
+                            nflag_dev, s);
 }
 
-int flat_rank_fallback_slices(int nq, int n, int d, int k) {
-    if (!flat_rank_ok(d, k)) return 0;
+int flat_rank_fallback_slices(int nq, int n, int k) {
     int tps, ib;
     return flat_rank_splits(nq, n, flat_rank_keep(k), &tps, &ib);
 }
@@ -877,14 +970,14 @@ void launch_flat_fallback(const uint32_t* flag_list, int nflag, const float* Q, 
         const int nf = nflag - f0 < 65535 ? nflag - f0 : 65535;
         hipLaunchKernelGGL(flat_exact_slice_kernel, dim3(sl, nf), dim3(256), 0, s, flag_list + f0, Q, X, n, d,
                            k, metric, len, keys + (size_t)f0 * sl * k);
-        hipLaunchKernelGGL(flat_exact_finish_kernel, dim3(nf), dim3(256), 0, s, flag_list + f0, sl, k,
-                           keys + (size_t)f0 * sl * k, out_idx, out_dist, nullptr);
+        launch_exact_finish(nf, flag_list + f0, sl, k, keys + (size_t)f0 * sl * k, out_idx, out_dist,
+                            nullptr, s);
     }
 }
 
 
-size_t flat_partial_count(int nq, int n, int d, int k) {
-    if (flat_rank_ok(d, k)) {
+size_t flat_partial_count(int nq, int n, int k, bool rank) {
+    if (rank) {
         int tps, ib;
         const int kk = flat_rank_keep(k);
         const size_t slots = (size_t)nq * flat_rank_splits(nq, n, kk, &tps, &ib);
@@ -893,19 +986,19 @@ size_t flat_partial_count(int nq, int n, int d, int k) {
     return (size_t)nq * flat_splits(nq, n, flat_keep(k)) * flat_keep(k);
 }
 
-size_t flat_pack_chunks(int n, int d) { return d <= 128 ? coarse_bf16_pack_chunks(n, d) : 0; }
+size_t flat_pack_chunks(int n, int d) { return d <= FR_MAXD ? coarse_bf16_pack_chunks(n, d) : 0; }
 
 void launch_flat_pack(const float* X, int n, int d, uint4* Xb, hipStream_t s) {
-    if (d <= 128 && n > 0) launch_coarse_bf16_pack(X, n, d, Xb, s);
+    if (d <= FR_MAXD && n > 0) launch_coarse_bf16_pack(X, n, d, Xb, s);
 }
 
-template <int DT>
+template <int DT, int J>
 static void launch_rank(const float* Q, int nq, int d, const uint4* Xb, const float* Xnorm, int n, int metric,
                         int kk, int tps, int ib, int sp, uint64_t* partial, uint32_t* pbound, hipStream_t s) {
     const size_t lds = 2 * (size_t)FR_TPS * 2 * DT * 64 * 16 + 2 * FR_TPS * 16 * 4;
-    ensure_dyn_lds((const void*)flat_rank_kernel<DT>, lds);
+    ensure_dyn_lds((const void*)flat_rank_kernel<DT, J>, lds);
     dim3 grid((nq + FR_ROWS - 1) / FR_ROWS, sp);
-    hipLaunchKernelGGL(flat_rank_kernel<DT>, grid, dim3(VGPU_BLOCK), lds, s, Q, nq, d, Xb, Xnorm, n, metric, kk,
+    hipLaunchKernelGGL((flat_rank_kernel<DT, J>), grid, dim3(VGPU_BLOCK), lds, s, Q, nq, d, Xb, Xnorm, n, metric, kk,
                        tps, ib, sp, partial, pbound);
 }
 
@@ -915,31 +1008,41 @@ void launch_flat_search(const float* Q, const float* Qsq, int nq, const float* X
                         unsigned int* overflow, uint32_t* flag_list, uint32_t* fbv, hipStream_t s,
                         hipEvent_t ranked) {
     if (nq <= 0) return;
-    if (Xb && flat_rank_ok(d, k)) {
+    if (Xb) {
         int tps, ib;
         const int kk = flat_rank_keep(k), sp = flat_rank_splits(nq, n, kk, &tps, &ib);
         uint32_t* pbound = reinterpret_cast<uint32_t*>(partial + (size_t)nq * sp * kk);
+#define FR_LAUNCH(DT)                                                                                       \
+    case DT:                                                                                                \
+        if (k <= 32) launch_rank<DT, fr_keys(32)>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); \
+        else launch_rank<DT, FR_J_WIDE>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); \
+        break;
         switch ((d + 31) / 32) {
-            case 1: launch_rank<1>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); break;
-            case 2: launch_rank<2>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); break;
-            case 3: launch_rank<3>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); break;
-            default: launch_rank<4>(Q, nq, d, Xb, Xnorm, n, metric, kk, tps, ib, sp, partial, pbound, s); break;
+            FR_LAUNCH(1)
+            FR_LAUNCH(2)
+            FR_LAUNCH(3)
+            FR_LAUNCH(4)
+            FR_LAUNCH(5)
+            FR_LAUNCH(6)
+            FR_LAUNCH(7)
+            FR_LAUNCH(8)
         }
+#undef FR_LAUNCH
         if (ranked) (void)hipEventRecord(ranked, s);
         const int tot = sp * kk;
         const dim3 mg((nq + 3) / 4);
-        if (tot <= 256)
-            hipLaunchKernelGGL(flat_merge_wave_kernel<4>, mg, dim3(256), 0, s, partial, pbound, sp, kk, Q, Qsq, X,
-                               nq, d, k, metric, xmax, ib, out_idx, out_dist, overflow, flag_list, fbv);
-        else if (tot <= 512)
-            hipLaunchKernelGGL(flat_merge_wave_kernel<8>, mg, dim3(256), 0, s, partial, pbound, sp, kk, Q, Qsq, X,
-                               nq, d, k, metric, xmax, ib, out_idx, out_dist, overflow, flag_list, fbv);
-        else if (tot <= 1024)
-            hipLaunchKernelGGL(flat_merge_wave_kernel<16>, mg, dim3(256), 0, s, partial, pbound, sp, kk, Q, Qsq,
-                               X, nq, d, k, metric, xmax, ib, out_idx, out_dist, overflow, flag_list, fbv);
-        else
-            hipLaunchKernelGGL(flat_merge_wave_kernel<32>, mg, dim3(256), 0, s, partial, pbound, sp, kk, Q, Qsq,
-                               X, nq, d, k, metric, xmax, ib, out_idx, out_dist, overflow, flag_list, fbv);
+#define FM_LAUNCH(E, R)                                                                                     \
+    hipLaunchKernelGGL((flat_merge_wave_kernel<E, R>), mg, dim3(256), 0, s, partial, pbound, sp, kk, Q, Qsq, X, nq, \
+                       d, k, metric, xmax, ib, out_idx, out_dist, overflow, flag_list, fbv)
+        if (k > 32) {
+            if (tot <= 768) FM_LAUNCH(12, 512);
+            else if (tot <= 1536) FM_LAUNCH(24, 512);
+            else FM_LAUNCH(48, 512);
+        } else if (tot <= 256) FM_LAUNCH(4, 256);
+        else if (tot <= 512) FM_LAUNCH(8, 256);
+        else if (tot <= 1024) FM_LAUNCH(16, 256);
+        else FM_LAUNCH(32, 256);
+#undef FM_LAUNCH
         return;
     }
     const int kk = flat_keep(k), cap = flat_cap(kk), sp = flat_splits(nq, n, kk);

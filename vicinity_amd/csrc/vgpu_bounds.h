@@ -84,4 +84,14 @@ __host__ __device__ inline float flat_bf16_tau(int d, int metric, float qn, floa
                    (float)(d + 1) * u * s * s) + pack + 1e-30f;
 }
 
+// The same for the score before packing, up to a constant of the query, when
+// the accumulator of metric 0 starts from about ||q||^2: each of the 3 dp
+// products (dp <= d + 31) then rounds a sum up to ||q||^2 larger (within 2u of
+// it), and so does the addition of ||x||^2.
+__host__ __device__ inline float flat_key_tau(int d, int metric, float qn, float xn) {
+    const float u = 5.9604645e-08f;
+    const float t = flat_bf16_tau((d + 31) / 32 * 32, metric, qn, xn, 0);
+    return metric == 0 ? t + (7.0f * (float)(d + 31) + 4.0f) * u * qn * qn : t;
+}
+
 }  // namespace vgpu

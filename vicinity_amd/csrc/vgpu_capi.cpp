@@ -654,9 +654,9 @@ int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float* out_bf16x3, fl
 
 int vgpu_test_bound_flat(size_t d, int metric, float qn, float xn, int ib, float* out) {
     return guard([&] {
-        need(out && d && (metric == 0 || metric == 1) && ib >= 0 && ib < 24,
+        need(out && d && (metric == 0 || metric == 1) && ib >= -1 && ib < 24,
              VGPU_ERR_INVALID_PARAMETER, "bad argument");
-        *out = vgpu::flat_bf16_tau((int)d, metric, qn, xn, ib);
+        *out = ib < 0 ? vgpu::flat_key_tau((int)d, metric, qn, xn) : vgpu::flat_bf16_tau((int)d, metric, qn, xn, ib);
     });
 }
 

@@ -30,12 +30,16 @@ void FlatIndex::add(const float* x, size_t count) {
     if (n + count >= 0xffffffffull) throw Error(VGPU_ERR_INVALID_PARAMETER, "more than 2^32-1 vectors");
     const size_t n0 = n;
     const double xmax0 = xmax2;
+    const bool finite0 = finite;
     host.insert(host.end(), x, x + count * d);
+    double sum = 0.0;
     for (size_t i = 0; i < count; i++) {
         double t = 0.0;
         for (size_t j = 0; j < d; j++) t += (double)x[i * d + j] * x[i * d + j];
         xmax2 = std::max(xmax2, t);
+        sum += t;
     }
+    finite = finite && std::isfinite(sum);  // squares of floats: no overflow in double
     n += count;
     try {
         sync_device();
@@ -45,6 +49,7 @@ void FlatIndex::add(const float* x, size_t count) {
         host.resize(n0 * d);
         n = n0;
         xmax2 = xmax0;
+        finite = finite0;
         try {
             sync_device();
         } catch (...) {
@@ -82,9 +87,26 @@ void FlatIndex::search_device(const float* d_q, size_t nq, size_t k, int64_t* d_
         VGPU_HIP(hipStreamSynchronize(s));
         return;
     }
+    const bool rank = d_xb.n && flat_rank_ok((int)d, (int)k, finite && xmax2 < 1e30);
+    const size_t step = rank && k > 32 ? (size_t)flat_rank_chunk() : nq;
+    float gemm = 0.f, total = 0.f;
+    unsigned int fb = 0;
+    for (size_t q0 = 0; q0 < nq; q0 += step) {
+        search_pass(d_q + q0 * d, std::min(step, nq - q0), k, rank, d_ids + q0 * k, d_dists + q0 * k, s);
+        gemm += ms_gemm;
+        total += ms_total;
+        fb += fallbacks;
+    }
+    ms_gemm = gemm;
+    ms_total = total;
+    fallbacks = fb;
+}
+
+void FlatIndex::search_pass(const float* d_q, size_t nq, size_t k, bool rank, int64_t* d_ids, float* d_dists,
+                            hipStream_t s) {
     const float xmax = (float)(std::sqrt(xmax2) * 1.0001 + 1e-30);
     w_qnorm.reserve(nq);
-    w_partial.reserve(flat_partial_count((int)nq, (int)n, (int)d, (int)k));
+    w_partial.reserve(flat_partial_count((int)nq, (int)n, (int)k, rank));
     w_idx.reserve(nq * k);
     w_dist.reserve(nq * k);
     w_overflow.reserve(1);
@@ -92,10 +114,10 @@ void FlatIndex::search_device(const float* d_q, size_t nq, size_t k, int64_t* d_
     w_fb.reserve(nq);
     VGPU_HIP(hipMemsetAsync(w_overflow.p, 0, sizeof(unsigned int), s));
     // the bf16x3 ranking path computes the query norms in its merge
-    const int rsl = d_xb.n ? flat_rank_fallback_slices((int)nq, (int)n, (int)d, (int)k) : 0;
+    const int rsl = rank ? flat_rank_fallback_slices((int)nq, (int)n, (int)k) : 0;
     if (!rsl) launch_flat_norms(d_q, (int)nq, (int)d, w_qnorm.p, s);
     VGPU_HIP(hipEventRecord(ev[0], s));
-    launch_flat_search(d_q, rsl ? nullptr : w_qnorm.p, (int)nq, d_x.p, d_xb.n ? d_xb.p : nullptr, d_xnorm.p,
+    launch_flat_search(d_q, rsl ? nullptr : w_qnorm.p, (int)nq, d_x.p, rank ? d_xb.p : nullptr, d_xnorm.p,
                        (int)n, (int)d, (int)k, metric, xmax, w_partial.p, w_idx.p, w_dist.p, w_overflow.p, w_flag.p,
                        w_fb.p, s, ev[3]);
     // the unproved queries (rare): exact scans over many workgroups.  The

@@ -316,13 +316,17 @@ void launch_fastscan_test(const uint8_t* packed, int n, int M, const float* lut,
 
 // Flat exact search.
 void launch_flat_norms(const float* X, int n, int d, float* norms, hipStream_t s);
-size_t flat_partial_count(int nq, int n, int d, int k);
-// bf16 hi/lo copy of the database for the ranking kernel (d <= 128; 0 chunks
+size_t flat_partial_count(int nq, int n, int k, bool rank);
+// Whether the bf16x3 ranking path takes this shape (plain_rows: every row
+// finite and of norm below 1e15), and its queries per pass above k 32.
+bool flat_rank_ok(int d, int k, bool plain_rows);
+int flat_rank_chunk();
+// bf16 hi/lo copy of the database for the ranking kernel (d <= 256; 0 chunks
 // otherwise), in the coarse quantiser's tile-major layout.
 size_t flat_pack_chunks(int n, int d);
 void launch_flat_pack(const float* X, int n, int d, uint4* Xb, hipStream_t s);
 // Qsq / Xnorm: squared norms (flat_norms); xmax: max ||x||; Xb: the packed
-// copy (null: the fp32 ranking path for every shape); `ranked` (optional) is
+// copy (null: the fp32 ranking path); `ranked` (optional) is
 // recorded between the ranking kernel and the merge.
 // Queries whose kept candidates cannot be proved to hold the exact top-k are
 // appended to flag_list (*overflow, zero on entry, counts them) and their
@@ -337,9 +341,8 @@ void launch_flat_search(const float* Q, const float* Qsq, int nq, const float* X
 // The bf16x3 ranking path's fallback for the nflag queries of flag_list
 // (fbv: their rescoring thresholds, written by the merge): only the slices
 // whose bound does not clear the threshold are scanned exhaustively.  keys:
-// scratch of nflag * flat_rank_fallback_slices(...) * k entries; 0 slices =
-// the ranking path is not used for this shape.
-int flat_rank_fallback_slices(int nq, int n, int d, int k);
+// scratch of nflag * flat_rank_fallback_slices(...) * k entries.
+int flat_rank_fallback_slices(int nq, int n, int k);
 void launch_flat_rank_fallback(const uint32_t* flag_list, int nflag, const uint32_t* fbv,
                                const uint64_t* partial, int nq, int n, int d, int k, int metric,
                                const float* Q, const float* X, uint64_t* keys, uint32_t* out_idx,

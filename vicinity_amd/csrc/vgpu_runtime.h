@@ -291,13 +291,14 @@ struct FlatIndex {
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {};
     DevBuf<float> d_x, d_xnorm, w_q, w_dist, w_odist, w_qnorm;
-    DevBuf<uint4> d_xb;  // bf16 hi/lo copy for the ranking kernel (d <= 128)
+    DevBuf<uint4> d_xb;  // bf16 hi/lo copy for the ranking kernel (d <= 256)
     DevBuf<uint64_t> w_partial, w_fbkeys;
     DevBuf<uint32_t> w_idx, w_flag, w_fb;
     DevBuf<int64_t> w_ids;
     DevBuf<unsigned int> w_overflow;
     std::vector<float> host;
     double xmax2 = 0.0;  // max ||x||^2
+    bool finite = true;  // no row holds a NaN or an infinity
     float ms_gemm = 0.f, ms_total = 0.f;
     unsigned int fallbacks = 0;  // queries of the last search that took the exhaustive exact scan
     bool stale = false;  // a failed add could not restore the device copy of the n rows
@@ -310,6 +311,11 @@ struct FlatIndex {
     void sync_device();  // device copy, norms and bf16 pack of host rows 0..n
     void search_device(const float* d_q, size_t nq, size_t k, int64_t* d_ids, float* d_dists,
                        hipStream_t s);
+
+  private:
+    // One pass: the ranking path's (rank) queries are bounded by flat_rank_chunk.
+    void search_pass(const float* d_q, size_t nq, size_t k, bool rank, int64_t* d_ids, float* d_dists,
+                     hipStream_t s);
 };
 
 // A file descriptor closed with its owner (also when a constructor throws).
