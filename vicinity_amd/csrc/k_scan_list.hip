@@ -147,7 +147,8 @@ __global__ __launch_bounds__(1024) void list_count_kernel(DevIndex ix, ScanArgs 
         for (int s0 = 0; s0 < a.P; s0 += 64) {
             const int s = s0 + lane;
             const uint32_t l = s < a.P ? pr[s] : 0u;
-            const uint32_t len = s < a.P ? ix.offsets[l + 1] - ix.offsets[l] : 0u;
+            // no such list: scanned as empty
+            const uint32_t len = s < a.P && l < (uint32_t)ix.L ? ix.offsets[l + 1] - ix.offsets[l] : 0u;
             const uint32_t nt = (len + 15) >> 4;
             uint32_t inc = nt;
             for (int o = 1; o < 64; o <<= 1) {
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(256) void list_scatter_kernel(DevIndex ix, ScanArgs
     if (i >= (uint32_t)a.nq * (uint32_t)a.P) return;
     const uint32_t q = i / (uint32_t)a.P, s = i % (uint32_t)a.P;
     const uint32_t l = a.probe[i];
-    if (ix.offsets[l + 1] == ix.offsets[l]) return;
+    if (l >= (uint32_t)ix.L || ix.offsets[l + 1] == ix.offsets[l]) return;
     const uint32_t word = q << SL_SLOT_BITS | s, pos = w.pos[i];
     const size_t o = (size_t)(q / (uint32_t)w.qw) * ix.L + l;
     w.pairs[w.first[o] + (pos & 0xffffu)] = word;
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(NTH) void list_final_kernel(DevIndex ix, ScanArgs a
     for (int i = tid; i < 256; i += NTH) hist[i] = 0u;
     for (int j = tid; j < d; j += NTH) sq[j] = a.qn[(size_t)q * d + j];
     for (int s = tid; s < P; s += NTH) {
-        const uint32_t l = a.probe[(size_t)q * P + s];
+        const uint32_t l = min(a.probe[(size_t)q * P + s], (uint32_t)ix.L - 1u);
         slist[s] = l;
         soff[s] = ix.offsets[l];
         stau[s] = list_tau(32 * w.sh.KT, M, ix.ds, w.t0[(size_t)q * P + s], ix.rmax);
@@ -1093,10 +1094,11 @@ __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs 
         __syncthreads();
         if (tid == 0) cnt = 0u;
         for (int p = tid; p < a.P; p += VGPU_BLOCK) {
-            const uint32_t l = pr[p], o = ix.offsets[l];
+            const bool in = pr[p] < (uint32_t)ix.L;
+            const uint32_t l = in ? pr[p] : 0u, o = ix.offsets[l];
             sl_l[p] = l;
             sl_o[p] = o;
-            sl_n[p] = ix.offsets[l + 1] - o;
+            sl_n[p] = in ? ix.offsets[l + 1] - o : 0u;
         }
         __syncthreads();
         SlTop top{keys, &cnt, ~0ull};
