@@ -254,8 +254,8 @@ def run_ivfpq(args, w):
     v._lib.check(v._lib.load().vgpu_test_scan_route(ix._h, nq, k, nprobe, pool or 0, ctypes.byref(route)))
     if route.value:
         # the whole scan by inverted list (pairs, sample, scores, rescoring) is
-        # timed as one; list_score_kernel is its largest part
-        kernel, kname = "list_score_kernel", "scan_list"
+        # timed as one; the score kernel is its largest part
+        kernel, kname = ("fs_list_kernel" if K == 16 else "list_score_kernel"), "scan_list"
     elif K == 16:
         kernel, kname = "fastscan_kernel", "fastscan"
     elif exact:
@@ -348,7 +348,7 @@ def run_flat(args, w):
                   "dists_bitexact": bool(gpu_d[:ns].tobytes() == cd.tobytes())}
         log(f"cpu baseline {cqps:.0f} QPS on {threads} threads; parity {parity}")
     config = {"workload": w.name, "n": n, "d": d, "k": k, "batch": nq, "metric": "l2"}
-    rank_bf16 = d <= 128 and k <= 32
+    rank_bf16 = d <= 256
     peak = BF16_PEAK_TFLOPS if rank_bf16 else FP32_PEAK_TFLOPS
     line = base_line(args, f"flat exact top-{k} QPS, {w.name} batch {nq // 1000}k; ranking GEMM "
                            f"TFLOP/s vs {'bf16' if rank_bf16 else 'fp32'} MFMA peak", qps, "queries/s",

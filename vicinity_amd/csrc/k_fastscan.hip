@@ -236,10 +236,8 @@ struct FsList {
     int slot = 0;
 };
 
-__global__ __launch_bounds__(256, 6) void fastscan_kernel(DevIndex ix, ScanArgs a, int wbuf) {
-    extern __shared__ __align__(16) char smem[];
-    const int q = blockIdx.x;
-    if (q >= a.nq) return;
+template <bool FLAGGED>
+__device__ __forceinline__ void fastscan_query(const DevIndex& ix, const ScanArgs& a, int wbuf, char* smem, int q) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar
     const int d = ix.d, M = ix.M, ds = ix.ds, P = a.P;
@@ -394,13 +392,31 @@ __global__ __launch_bounds__(256, 6) void fastscan_kernel(DevIndex ix, ScanArgs 
     for (int i = (int)*tk.count + lane; i < wbuf; i += 64) tk.keys[i] = ~0ull;
     if (lane == 0) cnt[4 + wave] = scanned;
     __syncthreads();
-    if (tid == 0) {
+    if (!FLAGGED && tid == 0) {
         uint32_t* st = a.qstat + (size_t)q * QSTAT_WORDS;
         st[0] = cnt[4] + cnt[5] + cnt[6] + cnt[7];
         st[1] = st[2] = st[3] = 0u;
     }
     block_bitonic_sort_keys(allkeys, 4 * wbuf);
     for (int j = tid; j < a.kout; j += blockDim.x) scan_emit(a, q, j, allkeys[j], allkeys[j] != ~0ull);
+}
+
+__global__ __launch_bounds__(256, 6) void fastscan_kernel(DevIndex ix, ScanArgs a, int wbuf) {
+    extern __shared__ __align__(16) char smem[];
+    const int q = blockIdx.x;
+    if (q >= a.nq) return;
+    fastscan_query<false>(ix, a, wbuf, smem, q);
+}
+
+// The queries the scan by inverted list left over (a.flag_list), the count
+// read on the device; their statistics stay.
+__global__ __launch_bounds__(256) void fastscan_flagged_kernel(DevIndex ix, ScanArgs a, int wbuf) {
+    extern __shared__ __align__(16) char smem[];
+    const uint32_t n = *a.flag_count;
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        fastscan_query<true>(ix, a, wbuf, smem, (int)a.flag_list[i]);
+        __syncthreads();  // the LDS is the next query's
+    }
 }
 
 size_t fastscan_lds_bytes(const DevIndex& ix, const ScanArgs& a) {
@@ -413,6 +429,14 @@ void launch_fastscan(const DevIndex& ix, const ScanArgs& a, hipStream_t s) {
     size_t lds = fastscan_lds_bytes(ix, a);
     ensure_dyn_lds((const void*)fastscan_kernel, lds);
     hipLaunchKernelGGL(fastscan_kernel, dim3(a.nq), dim3(VGPU_BLOCK), lds, s, ix, a,
+                       fs_wave_buf(a.kout));
+}
+
+void launch_fastscan_flagged(const DevIndex& ix, const ScanArgs& a, hipStream_t s) {
+    if (a.nq <= 0) return;
+    const size_t lds = fastscan_lds_bytes(ix, a);
+    ensure_dyn_lds((const void*)fastscan_flagged_kernel, lds);
+    hipLaunchKernelGGL(fastscan_flagged_kernel, dim3(a.nq < 512 ? a.nq : 512), dim3(VGPU_BLOCK), lds, s, ix, a,
                        fs_wave_buf(a.kout));
 }
 

@@ -64,7 +64,6 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 #define SL_WAVES 8
 #define SL_THREADS (64 * SL_WAVES)
 #define SL_STAGE 320                // survivors a wave stages in LDS before it flushes
-#define SL_SEG 16                   // entry tiles (16 entries each) per work item, at least
 #define SL_MAXSEG 16                // segments per list, at most
 
 // Padded shape of the score product: dsp dimensions per codebook in the MFMA
@@ -181,9 +180,9 @@ __global__ __launch_bounds__(1024) void list_count_kernel(DevIndex ix, ScanArgs 
     for (int l = tid; l < ix.L; l += 1024) out[l] = hist[l];
 }
 
-// Segments of a list of nt tiles: SL_SEG tiles each, at most SL_MAXSEG.
-__device__ __forceinline__ uint32_t sl_segs(uint32_t nt) {
-    return min((nt + SL_SEG - 1) / SL_SEG, (uint32_t)SL_MAXSEG);
+// Segments of a list of nt tiles: seg tiles each, at most SL_MAXSEG.
+__device__ __forceinline__ uint32_t sl_segs(uint32_t nt, uint32_t seg) {
+    return min((nt + seg - 1) / seg, (uint32_t)SL_MAXSEG);
 }
 
 // 256 lists per workgroup, four threads each (a quarter of the counting
@@ -221,7 +220,7 @@ __global__ __launch_bounds__(1024) void list_plan_kernel(DevIndex ix, ListWs w) 
             c[ph] += part[ph][g][li];
         }
         nb[ph] = (c[ph] + SL_PAIRS - 1) / SL_PAIRS;
-        ns[ph] = sl_segs(ph ? nt : min(nt, (uint32_t)w.tcap));
+        ns[ph] = sl_segs(ph ? nt : min(nt, (uint32_t)w.tcap), (uint32_t)w.seg);
         v[2 * ph] = c[ph];
         v[2 * ph + 1] = nb[ph] * ns[ph];
     }
@@ -1203,10 +1202,8 @@ static void launch_rescue(const DevIndex& ix, const ScanArgs& a, const ListWs& w
     hipLaunchKernelGGL(k, dim3(SL_RESCUE), dim3(VGPU_BLOCK), lds, s, ix, a, w);
 }
 
-void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& ws, hipStream_t s) {
-    if (a.nq <= 0) return;
-    ListWs w = ws;
-    w.rows = w.padded ? w.padded : a.qn;
+// The pairs and work items of a chunk.
+void launch_list_pairs(const DevIndex& ix, const ScanArgs& a, ListWs& w, hipStream_t s) {
     w.qw = list_count_queries(a.nq);
     w.nwg = (a.nq + w.qw - 1) / w.qw;
     launch_zero_words(reinterpret_cast<unsigned long long*>(w.heads), 2 + SL_RESCUE / 2, s);
@@ -1216,13 +1213,24 @@ void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& ws, h
     hipLaunchKernelGGL(list_plan_kernel, dim3((ix.L + 255) / 256), dim3(1024), 0, s, ix, w);
     const size_t np = (size_t)a.nq * a.P;
     hipLaunchKernelGGL(list_scatter_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, ix, a, w);
-    launch_score_any(ix, a, w, true, s);
+}
+
+void launch_list_bound(const ScanArgs& a, const ListWs& w, hipStream_t s) {
     const dim3 bg((a.nq + 3) / 4);
     switch (w.tcap) {
-        case 16: hipLaunchKernelGGL(list_bound_kernel<1>, bg, dim3(256), 0, s, a, w); break;
         case 32: hipLaunchKernelGGL(list_bound_kernel<2>, bg, dim3(256), 0, s, a, w); break;
-        default: hipLaunchKernelGGL(list_bound_kernel<4>, bg, dim3(256), 0, s, a, w); break;
+        case 64: hipLaunchKernelGGL(list_bound_kernel<4>, bg, dim3(256), 0, s, a, w); break;
+        default: hipLaunchKernelGGL(list_bound_kernel<8>, bg, dim3(256), 0, s, a, w); break;
     }
+}
+
+void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& ws, hipStream_t s) {
+    if (a.nq <= 0) return;
+    ListWs w = ws;
+    w.rows = w.padded ? w.padded : a.qn;
+    launch_list_pairs(ix, a, w, s);
+    launch_score_any(ix, a, w, true, s);
+    launch_list_bound(a, w, s);
     launch_score_any(ix, a, w, false, s);
     if (a.kout <= 16) launch_final<64>(ix, a, w, s);
     else launch_final<256>(ix, a, w, s);

@@ -612,6 +612,11 @@ static uint32_t host_bf16(float x) {
 // that squared norms could overflow, leave the index without it.
 void IvfpqIndex::upload_list_scan() {
     lshape = list_shape((int)d, (int)M, (int)K, (int)ds);
+    if (K == 16) {  // the 4-bit scan by list (k_fast_list.hip): nibbles, no table
+        lshape.LW = fast_list_words((int)M);
+        lshape.contig = true;
+        lshape.ok = fast_list_shape((int)M, (int)ds);
+    }
     max_list = 0;
     for (size_t l = 0; l < L; l++) max_list = std::max<uint32_t>(max_list, (uint32_t)(offsets[l + 1] - offsets[l]));
     // the score kernel's buffer loads take 32-bit byte offsets
@@ -628,6 +633,18 @@ void IvfpqIndex::upload_list_scan() {
         d_lbias.release();
         d_lcent.release();
         d_dimmap.release();
+        return;
+    }
+    if (K == 16) {
+        std::vector<uint32_t> off(L + 1, 0);
+        for (size_t l = 0; l < L; l++) off[l + 1] = off[l] + (uint32_t)((offsets[l + 1] - offsets[l] + 15) / 16);
+        d_ltoff.upload(off.data(), L + 1, stream);
+        d_lcodes.reserve((size_t)off[L] * 64 * lshape.LW);
+        dix.ltoff = d_ltoff.p;
+        dix.ltiles = off[L];
+        dix.lcodes = d_lcodes.p;
+        launch_fast_list_tiles(dix, d_lcodes.p, stream);
+        VGPU_HIP(hipStreamSynchronize(stream));  // before the host array goes
         return;
     }
     const int dsp = lshape.dsp, parts = lshape.parts, Mt = lshape.KT * 32 / dsp;
@@ -762,7 +779,7 @@ vgpu_search_stats IvfpqIndex::last_stats() {
 // 128, 0.8M 166 -> 154, 8M 309 -> 202.  A few wide codebooks cost few lookups
 // and many products: 300k x 96, M 8, 38M 208 -> 285.
 static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
-    if (!ix.lshape.ok || ix.mode != VGPU_MODE_FAST || pl.wide || pl.P == 0 || pl.kout > 256 || ix.L > SL_MAX_LISTS ||
+    if (!ix.lshape.ok || (ix.K != 16 && ix.mode != VGPU_MODE_FAST) || pl.wide || pl.P == 0 || pl.kout > 256 || ix.L > SL_MAX_LISTS ||
         (pl.opq && !ix.lshape.contig))
         return false;
     int sb = 0;
@@ -770,6 +787,25 @@ static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
     pl.tbits = std::min(26, 32 - sb);
     if (ix.max_list >= (1u << pl.tbits)) return false;
     const double pairs = (double)nq * pl.P, lookups = pairs * ix.n() / ix.L * ix.M;
+    if (ix.K == 16) {
+        // The 4-bit scan by list costs about 120 us of launches and sampling
+        // above fastscan_kernel's and less per entry; both build a table per
+        // pair, so lists must be long enough for the entries to matter, less so
+        // at a large k, which slows fastscan_kernel's wave buffers.  Whole
+        // search, fastscan -> by list, k 10 / k 100: M 50, 488 per list, 9M
+        // entries 341 -> 310 / 413 -> 333 us, 31M 446 -> 400 / 518 -> 448, 313M
+        // 2292 -> 1054 / 2615 -> 1153; M 25, 586 per list, 28M 281 -> 318 / 394 ->
+        // 361, 94M 677 -> 464 / 1031 -> 535; M 16, 390 per list, 9M 157 -> 231 /
+        // 245 -> 256, 31M 347 -> 275 / 614 -> 309; M 50, 195 per list, 31M 589 ->
+        // 662 / 827 -> 667; M 64, 122 per list, 12M 424 -> 465 / 550 -> 499, 39M
+        // 1055 -> 984 / 1361 -> 1001.
+        const double entries = pairs * ix.n() / ix.L;
+        const bool large_k = pl.kout >= 64;
+        if (pairs < 16.0 * ix.L || entries < (large_k ? 25e6 : 30e6) || ix.n() < (large_k ? 96 : 256) * ix.L) return false;
+        pl.tcap = 128;
+        pl.cap = 6144;
+        return true;
+    }
     if (pairs < 1.5 * ix.L) return false;
     if (pl.opq) {
         if (lookups < 0.02e9) return false;
@@ -874,6 +910,7 @@ size_t IvfpqIndex::ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) c
         const size_t np = c * pl.P, ni = list_max_items(c, pl.P, L);
         lw.sh = lshape;
         lw.tcap = pl.tcap;
+        if (K == 16) lw.seg = 64;
         lw.cap = pl.cap;
         lw.rcap = pl.rcap;
         lw.tbits = pl.tbits;
@@ -1039,7 +1076,8 @@ void IvfpqIndex::run_search(const float* d_q, size_t nq, const SearchPlan& pl, c
         a.rres = pl.opq ? w.rres : nullptr;
         if (K == 16) {
             a.kk = (int)kout;
-            launch_fastscan(dix, a, s);
+            if (pl.list) launch_fast_list(dix, a, w.list, s);
+            else launch_fastscan(dix, a, s);
             if (allp) VGPU_HIP(hipEventRecord(ev[4], s));
             if (scanp) VGPU_HIP(hipEventRecord(ws->sev[4 * ci + 1], s));
         } else if (pl.list) {

@@ -183,7 +183,6 @@ struct ListShape {
 };
 ListShape list_shape(int d, int M, int K, int ds);
 #define SL_SLOT_BITS 10   // probe slots of a pair word (the rest: query of the chunk)
-#define SL_TCAP_MAX 160   // sample tiles per query, at most
 // Queries each workgroup of the pair count takes: at most 96 workgroups, whose
 // counts of every list are kept apart.
 #define SL_COUNT_WG 96
@@ -196,7 +195,8 @@ inline int list_count_queries(int nq) {
 // Device workspace of one chunk (sizes in ws_layout).
 struct ListWs {
     ListShape sh;
-    int tcap = 0;   // sample tiles per query
+    int tcap = 0;   // sample tiles per query: 32, 64 or 128
+    int seg = 16;   // entry tiles (16 entries each) per work item, at least
     int cap = 0;    // survivors per query
     int rcap = 0;   // rescored survivors per query
     int tbits = 0;  // entry bits of a survivor's label (slot << tbits | entry)
@@ -230,6 +230,19 @@ void launch_list_tiles(const DevIndex& ix, const double* cwn, const ListShape& s
 // The whole scan of a chunk: rows written like launch_scan8_fast's; queries
 // whose survivors do not fit are appended to a.flag_list and scanned exhaustively.
 void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& w, hipStream_t s);
+// Its parts that the 4-bit scan by list shares: the pairs and work items
+// (sets w.qw and w.nwg), and the bound of each query's sample.
+void launch_list_pairs(const DevIndex& ix, const ScanArgs& a, ListWs& w, hipStream_t s);
+void launch_list_bound(const ScanArgs& a, const ListWs& w, hipStream_t s);
+
+// ---- 4-bit FastScan by inverted list (k_fast_list.hip) ----
+// Its shapes, and the code words per lane and tile of lcodes.
+bool fast_list_shape(int M, int ds);
+int fast_list_words(int M);
+void launch_fast_list_tiles(const DevIndex& ix, uint32_t* lcodes, hipStream_t s);
+void launch_fast_list(const DevIndex& ix, const ScanArgs& a, const ListWs& w, hipStream_t s);
+// fastscan_kernel for the queries of a.flag_list (*a.flag_count of them).
+void launch_fastscan_flagged(const DevIndex& ix, const ScanArgs& a, hipStream_t s);
 #define QSTAT_WORDS 4
 // Search statistics: entries scanned, fallbacks, flushes, appends, fallbacks
 // from ties, second passes; counter i lives at counters[i * COUNTER_STRIDE]
