@@ -30,23 +30,34 @@ __global__ __launch_bounds__(256) void normalize_kernel(const float* __restrict_
                                                         unsigned int* __restrict__ nbad) {
     extern __shared__ float srow[];  // [NR_ROWS][d + 1]
     __shared__ float snorm[NR_ROWS];
+    __shared__ uint32_t sbad[NR_ROWS];
     const int tid = threadIdx.x;
     const int r0 = blockIdx.x * NR_ROWS;
     const int rows = min(NR_ROWS, n - r0);
     const int st = d + 1;
     const float* src = x + (size_t)r0 * d;
-    for (int e = tid; e < rows * d; e += VGPU_BLOCK) srow[(e / d) * st + e % d] = src[e];
+    if (tid < NR_ROWS) sbad[tid] = 0u;
+    __syncthreads();
+    for (int e = tid; e < rows * d; e += VGPU_BLOCK) {
+        const float v = src[e];
+        srow[(e / d) * st + e % d] = v;
+        if ((__float_as_uint(v) & 0x7f800000u) == 0x7f800000u) sbad[e / d] = 1u;
+    }
     __syncthreads();
     if (tid < rows) {
         float* xr = srow + tid * st;
-        if (row_nonfinite(xr, d)) {
+        if (sbad[tid]) {
             for (int j = 0; j < d; j++) xr[j] = 0.0f;
             if (nbad) atomicAdd(nbad, 1u);
             if (qbad) qbad[r0 + tid] = 1u;
         } else if (qbad) {
             qbad[r0 + tid] = 0u;
         }
+        // the sum is one chain of adds (the reference's order); 16 reads of LDS
+        // are in flight under it (one at a time the chain waits for each: 42 us
+        // for 1000 rows of 768)
         float s = 0.0f;
+#pragma unroll 16
         for (int j = 0; j < d; j++) s = __fadd_rn(s, __fmul_rn(xr[j], xr[j]));
         const float nrm = sqrtf(s);
         snorm[tid] = nrm;
@@ -72,68 +83,91 @@ void launch_normalize(const float* x, float* out, float* norms, int n, int d, hi
 
 // ---- coarse GEMM --------------------------------------------------------
 // D[q][c] = sum_k Q[q][k] * C[c][k] with v_mfma_f32_16x16x4_f32.
-// Block tile 64 (queries) x 64 (centroids), 4 waves each own a 32x32 quarter
-// as 2x2 MFMA tiles.  Operand layout of 16x16x4 f32 (wave64): A[i][k] comes
+// Block tile T (queries) x T (centroids), 4 waves each own a quarter as
+// (T / 32)^2 MFMA tiles.  Operand layout of 16x16x4 f32 (wave64): A[i][k] comes
 // from lane i + 16k, B[k][j] from lane j + 16k, D[i][j] lands in lane
-// j + 16*(i/4), element i%4.
-#define CT_M 64
-#define CT_N 64
+// j + 16*(i/4), element i%4.  The next slab of CT_K dimensions is loaded into
+// registers under the products of this one; every dot product adds its
+// dimensions in the same order in both tile sizes.
 #define CT_K 32
 
+template <int T>
 __global__ __launch_bounds__(256) void coarse_dots_kernel(const float* __restrict__ Q,
                                                           const float* __restrict__ C,
                                                           float* __restrict__ D, int nq, int L,
                                                           int d) {
-    __shared__ float As[CT_M][CT_K + 1];
-    __shared__ float Bs[CT_N][CT_K + 1];
+    constexpr int NT = T / 32, PER = T * CT_K / 256;
+    __shared__ float As[T][CT_K + 1];
+    __shared__ float Bs[T][CT_K + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row0 = blockIdx.y * CT_M, col0 = blockIdx.x * CT_N;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    floatx4 acc00 = {0.f, 0.f, 0.f, 0.f}, acc01 = acc00, acc10 = acc00, acc11 = acc00;
+    const int row0 = blockIdx.y * T, col0 = blockIdx.x * T;
+    const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+    floatx4 acc[NT][NT];
+#pragma unroll
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
     const int li = lane & 15, lk = lane >> 4;
+    float pa[PER], pb[PER];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int e = i * 256 + tid, gk = k0 + e % CT_K, gr = row0 + e / CT_K, gc = col0 + e / CT_K;
+            pa[i] = (gr < nq && gk < d) ? Q[(size_t)gr * d + gk] : 0.0f;
+            pb[i] = (gc < L && gk < d) ? C[(size_t)gc * d + gk] : 0.0f;
+        }
+    };
+    fetch(0);
     for (int k0 = 0; k0 < d; k0 += CT_K) {
-        for (int e = tid; e < CT_M * CT_K; e += 256) {
-            int r = e / CT_K, c = e % CT_K;
-            int gk = k0 + c;
-            int gr = row0 + r, gc = col0 + r;
-            As[r][c] = (gr < nq && gk < d) ? Q[(size_t)gr * d + gk] : 0.0f;
-            Bs[r][c] = (gc < L && gk < d) ? C[(size_t)gc * d + gk] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int e = i * 256 + tid;
+            As[e / CT_K][e % CT_K] = pa[i];
+            Bs[e / CT_K][e % CT_K] = pb[i];
         }
         __syncthreads();
+        if (k0 + CT_K < d) fetch(k0 + CT_K);
 #pragma unroll
         for (int kk = 0; kk < CT_K; kk += 4) {
-            float a0 = As[wm + li][kk + lk];
-            float a1 = As[wm + 16 + li][kk + lk];
-            float b0 = Bs[wn + li][kk + lk];
-            float b1 = Bs[wn + 16 + li][kk + lk];
-            acc00 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc00, 0, 0, 0);
-            acc01 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc01, 0, 0, 0);
-            acc10 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc10, 0, 0, 0);
-            acc11 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc11, 0, 0, 0);
+            float a[NT], b[NT];
+#pragma unroll
+            for (int i = 0; i < NT; i++) {
+                a[i] = As[wm + 16 * i + li][kk + lk];
+                b[i] = Bs[wn + 16 * i + li][kk + lk];
+            }
+#pragma unroll
+            for (int i = 0; i < NT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
         }
         __syncthreads();
     }
-    const int rbase = row0 + wm + 4 * lk;
-    const int cbase = col0 + wn + li;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        int r0 = rbase + r, r1 = rbase + 16 + r;
-        if (r0 < nq) {
-            if (cbase < L) D[(size_t)r0 * L + cbase] = acc00[r];
-            if (cbase + 16 < L) D[(size_t)r0 * L + cbase + 16] = acc01[r];
+    for (int i = 0; i < NT; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = row0 + wm + 16 * i + 4 * lk + r;
+            if (row >= nq) continue;
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const int col = col0 + wn + 16 * j + li;
+                if (col < L) D[(size_t)row * L + col] = acc[i][j][r];
+            }
         }
-        if (r1 < nq) {
-            if (cbase < L) D[(size_t)r1 * L + cbase] = acc10[r];
-            if (cbase + 16 < L) D[(size_t)r1 * L + cbase + 16] = acc11[r];
-        }
-    }
 }
 
+// 64 x 64 tiles, or 32 x 32 below two workgroups of those per CU: 1000 queries
+// of 317 lists at 768 dimensions are 80 workgroups of 64 x 64, whose 24 slabs
+// each waited for their loads (135 us).
 void launch_coarse_dots(const float* Q, const float* C, float* D, int nq, int L, int d,
                         hipStream_t s) {
     if (nq <= 0 || L <= 0) return;
-    dim3 grid((L + CT_N - 1) / CT_N, (nq + CT_M - 1) / CT_M);
-    hipLaunchKernelGGL(coarse_dots_kernel, grid, dim3(256), 0, s, Q, C, D, nq, L, d);
+    auto tiles = [&](int t) { return dim3((L + t - 1) / t, (nq + t - 1) / t); };
+    if ((size_t)tiles(64).x * tiles(64).y >= 512)
+        hipLaunchKernelGGL(coarse_dots_kernel<64>, tiles(64), dim3(256), 0, s, Q, C, D, nq, L, d);
+    else
+        hipLaunchKernelGGL(coarse_dots_kernel<32>, tiles(32), dim3(256), 0, s, Q, C, D, nq, L, d);
 }
 
 // ---- probe selection ----------------------------------------------------
