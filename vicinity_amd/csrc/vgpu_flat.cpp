@@ -34,8 +34,13 @@ void FlatIndex::add(const float* x, size_t count) {
     host.insert(host.end(), x, x + count * d);
     double sum = 0.0;
     for (size_t i = 0; i < count; i++) {
-        double t = 0.0;
-        for (size_t j = 0; j < d; j++) t += (double)x[i * d + j] * x[i * d + j];
+        double p[4] = {0.0, 0.0, 0.0, 0.0};  // four chains: one waits for each add
+        const float* r = x + i * d;
+        size_t j = 0;
+        for (; j + 4 <= d; j += 4)
+            for (int c = 0; c < 4; c++) p[c] += (double)r[j + c] * r[j + c];
+        for (; j < d; j++) p[0] += (double)r[j] * r[j];
+        const double t = (p[0] + p[1]) + (p[2] + p[3]);
         xmax2 = std::max(xmax2, t);
         sum += t;
     }
