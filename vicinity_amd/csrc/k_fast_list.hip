@@ -32,8 +32,10 @@
 // Bounds, at 10k queries x 64 lists of 488 entries, M 50: the table build's
 // vector instructions and LDS reads (two passes over 800 values per pair, as in
 // fastscan_kernel), then the one-hot reads; the matrix cores are busy about
-// 100 of 870 us.  Whole search 2730 -> 1253 us.  The rows' parts of the next
-// step are loaded under the present one (1313 us without).
+// 100 of 830 us.  Whole search 2730 -> 1117 us.  The rows' parts of the next
+// step are loaded under the present one (1313 -> 1253), and items hold 32
+// pairs, one pass of a wave: with 64 the few popular lists' waves ran twice as
+// long at the end of the sample and of the scan (1253 -> 1117).
 #include "vgpu_device.h"
 #include "vgpu_launch.h"
 
@@ -441,12 +443,9 @@ __global__ __launch_bounds__(FL_THREADS, 2) void fs_list_kernel(DevIndex ix, Sca
         if (SAMPLE) nt = min(nt, (uint32_t)w.tcap);
         const uint32_t s0 = sg & 255u, nseg = sg >> 8, per = (nt + nseg - 1) / nseg;
         const uint32_t tile0 = min(s0 * per, nt), tile1 = min(tile0 + per, nt);
-        if (tile0 < tile1)
-            for (uint32_t h = 0; h < np; h += FL_PAIRS) {
-                const uint32_t n = min((uint32_t)FL_PAIRS, np - h);
-                const uint32_t word = pairs[p0 + h + min((uint32_t)lane, n - 1u)];
-                fl_item<KS, DS, LW, SAMPLE>(ix, a, w, cbs, onehot, sw, l, n, word, tile0, tile1);
-            }
+        if (tile0 < tile1)  // np <= FL_PAIRS
+            fl_item<KS, DS, LW, SAMPLE>(ix, a, w, cbs, onehot, sw, l, np, pairs[p0 + min((uint32_t)lane, np - 1u)], tile0,
+                                        tile1);
     }
 }
 

@@ -219,7 +219,7 @@ __global__ __launch_bounds__(1024) void list_plan_kernel(DevIndex ix, ListWs w) 
             if (g == quarter) before[ph] = c[ph];
             c[ph] += part[ph][g][li];
         }
-        nb[ph] = (c[ph] + SL_PAIRS - 1) / SL_PAIRS;
+        nb[ph] = (c[ph] + (uint32_t)w.ipairs - 1u) / (uint32_t)w.ipairs;
         ns[ph] = sl_segs(ph ? nt : min(nt, (uint32_t)w.tcap), (uint32_t)w.seg);
         v[2 * ph] = c[ph];
         v[2 * ph + 1] = nb[ph] * ns[ph];

@@ -907,10 +907,10 @@ size_t IvfpqIndex::ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) c
     if (pl.t2) carve(w.t2, c * M * K);
     if (pl.list) {
         ListWs& lw = w.list;
-        const size_t np = c * pl.P, ni = list_max_items(c, pl.P, L);
+        const size_t np = c * pl.P, ni = list_max_items(c, pl.P, L, K == 16 ? 32 : 64);
         lw.sh = lshape;
         lw.tcap = pl.tcap;
-        if (K == 16) lw.seg = 64;
+        if (K == 16) lw.seg = 64, lw.ipairs = 32;
         lw.cap = pl.cap;
         lw.rcap = pl.rcap;
         lw.tbits = pl.tbits;

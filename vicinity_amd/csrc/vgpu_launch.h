@@ -197,6 +197,7 @@ struct ListWs {
     ListShape sh;
     int tcap = 0;   // sample tiles per query: 32, 64 or 128
     int seg = 16;   // entry tiles (16 entries each) per work item, at least
+    int ipairs = 64;  // pairs per work item, at most (a multiple of 16)
     int cap = 0;    // survivors per query
     int rcap = 0;   // rescored survivors per query
     int tbits = 0;  // entry bits of a survivor's label (slot << tbits | entry)
@@ -222,8 +223,10 @@ struct ListWs {
     uint32_t* rescued = nullptr;  // [SL_RESCUE] finished workgroups of each flagged query
     uint64_t* rescue = nullptr;   // [SL_RESCUE kout] their keys
 };
-// Work items of a chunk of nq queries, at most: blocks of 64 pairs x 16 segments.
-inline size_t list_max_items(size_t nq, size_t P, size_t L) { return 16 * (nq * P / 64 + (L < nq * P ? L : nq * P)); }
+// Work items of a chunk of nq queries, at most: blocks of ipairs pairs x 16 segments.
+inline size_t list_max_items(size_t nq, size_t P, size_t L, size_t ipairs) {
+    return 16 * (nq * P / ipairs + (L < nq * P ? L : nq * P));
+}
 // lcodes / lbias of every list (cwn: |codeword|^2 in float64).
 void launch_list_tiles(const DevIndex& ix, const double* cwn, const ListShape& sh, uint32_t* lcodes, float* lbias,
                        hipStream_t s);
