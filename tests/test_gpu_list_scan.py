@@ -117,6 +117,29 @@ def test_equal_distances_beyond_the_buffers(oracle, copies, k):
     assert ix.last_stats()["fallback_queries"] >= 40
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("opq,d,M,K", [(False, 100, 25, 256), (True, 128, 16, 256), (True, 64, 16, 64)])
+def test_crowds_of_flagged_queries(oracle, opq, d, M, K):
+    """300 flagged queries in the first chunk and 20 in the second (16,384 a
+    chunk), of which list_rescue_kernel takes the 20 and the EXACT kernel the
+    300: 1500 equal entries are kept but not rescored, 6000 are not kept."""
+    rng = np.random.default_rng(d + M)
+    rot = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((d, d)))[0].astype(np.float32)) if opq else None
+    for copies in (1500, 6000):
+        _print_case(f"list scan: crowds of flagged queries, {copies} copies, d={d} M={M} ksub={K} opq={opq}")
+        x = rng.standard_normal((2000, d)).astype(np.float32)
+        x = np.concatenate([np.repeat(x[:1], copies, axis=0), x])
+        perm = rng.permutation(len(x))
+        ix, oix, _ = _index(oracle, rng, len(x), d, 16, M, K, rotation=rot, x=x[perm], together=perm < copies)
+        q = x[rng.integers(copies + 10, len(x), 16_450)]
+        q[np.concatenate([np.arange(0, 3000, 10), np.arange(16_400, 16_420)])] = x[0]
+        q = (q + 1e-3 * rng.standard_normal(q.shape)).astype(np.float32)
+        _same(ix, oix, q, 20, 16)
+        assert ix.last_stats()["fallback_queries"] >= 320
+        _same(ix, oix, q[:2000], 20, 16)
+        assert ix.last_stats()["fallback_queries"] >= 200
+
+
 @pytest.mark.parametrize("d,M,scale", [(32, 8, 1.0), (96, 48, 0.05), (128, 16, 30.0)])
 def test_error_bound(oracle, d, M, scale):
     """|a - e| <= list_tau with a from bf16x3 products in float32 (started

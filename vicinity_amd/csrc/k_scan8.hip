@@ -746,7 +746,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void scan8_filtered_kernel(DevInde
 }
 
 // FL = false: every query of the batch, block q taking query q.  FL = true:
-// the flagged queries the FAST kernel listed before this launch, the blocks
+// the flagged queries listed before this launch, the blocks
 // striding over the list.  Two kernels, each with one call site of the query
 // body: a loop over queries in the whole-batch kernel would keep the body's
 // per-lane addresses live across it (they are loop-invariant) and spill them
@@ -761,7 +761,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void scan8_exact_kernel(DevIndex i
         exact_query<MT, KT, CWD>(ix, a, buf, smem, (int)blockIdx.x, cw);
     } else {
         const uint32_t nf = *a.flag_count;
-        if (blockIdx.x >= nf) return;
+        if (blockIdx.x >= nf || nf <= (uint32_t)a.flag_over) return;
         load_codewords<MT, CWD>(ix, cw);
         for (uint32_t fi = blockIdx.x; fi < nf; fi += gridDim.x) {
             __syncthreads();
@@ -822,8 +822,10 @@ static void launch_mk(const DevIndex& ix, const ScanArgs& a, hipStream_t s) {
     auto k = a.only_flagged ? pick(std::true_type{}) : pick(std::false_type{});
     ensure_dyn_lds((const void*)k, lds);
     // Flagged queries: a small grid walks the list the FAST kernel wrote.
-    // flagged queries are rare: a small grid keeps the usual empty launch cheap
-    const int grid = a.only_flagged ? (a.nq < 64 ? a.nq : 64) : a.nq;
+    // flagged queries are rare: a small grid keeps the usual empty launch cheap.
+    // Where only a crowd of them comes here (flag_over): two workgroups per CU.
+    const int most = a.flag_over ? 512 : 64;
+    const int grid = a.only_flagged && a.nq > most ? most : a.nq;
     hipLaunchKernelGGL(k, dim3(grid), dim3(SCAN_THREADS), lds, s, ix, a, buf);
 }
 

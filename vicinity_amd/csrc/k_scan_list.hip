@@ -28,9 +28,10 @@
 // Scores are bf16x3 (r = rh + rl, y = yh + yl; rh.yh + rh.yl + rl.yh in
 // float32, v_mfma_f32_16x16x32_bf16) and every comparison allows for their
 // error bound list_tau, so the rescored set contains the reference's top k.
-// A query with more survivors than its buffer holds is flagged, like a FAST
-// query whose proof fails, and list_rescue_kernel scans its lists with the
-// reference's arithmetic.
+// A query with more survivors than its buffer holds, or more within the bound
+// than are rescored, is flagged, like a FAST query whose proof fails:
+// list_rescue_kernel, or for many of them the EXACT kernel, scores its entries
+// with the reference's arithmetic.
 //
 // Bounds, at 10k queries: the score kernel is held by the LDS codeword gathers
 // and the latency of the work items' prologues, at two waves per SIMD (the
@@ -137,6 +138,8 @@ __global__ __launch_bounds__(1024) void list_count_kernel(DevIndex ix, ScanArgs 
     extern __shared__ __align__(16) char smem[];
     uint32_t* hist = reinterpret_cast<uint32_t*>(smem);  // [L]
     const int tid = threadIdx.x, lane = tid & 63;
+    if (blockIdx.x == 0)  // heads, then rescued: first used by the kernels that follow
+        for (int i = tid; i < 4 + SL_RESCUE_MAX; i += 1024) w.heads[i] = 0u;
     for (int l = tid; l < ix.L; l += 1024) hist[l] = 0u;
     __syncthreads();
     const int q0 = blockIdx.x * w.qw, q1 = min(q0 + w.qw, a.nq);
@@ -1068,27 +1071,32 @@ __device__ __forceinline__ uint32_t sl_top_end(SlTop& t, int k) {
     return min(c, (uint32_t)k);
 }
 
-// The queries whose survivors did not fit, exhaustively with the reference's
-// arithmetic: each one's entries are spread over up to 64 workgroups, whose k
-// smallest keys the last of them to finish merges.  Rare (a query among lists
-// that are all far from it, or masses of equal distances); one workgroup per
-// query in the EXACT kernel took 380 us for a single query at 10M x 96.
+// Up to SL_RESCUE_MAX flagged queries with the reference's arithmetic: each
+// one's survivors, when its buffer holds them all, or else every entry of its
+// lists, spread over up to 64 workgroups whose k smallest keys the last of them
+// to finish merges.  One workgroup per query, as the EXACT kernel has it, took
+// 380 us for a single query at 10M x 96; but the entries here cost an L1 gather
+// per codeword (6 per ns), where the EXACT kernel looks them up in LDS (50 per
+// ns over a full chip), so more flagged queries than that are left to it.
 template <int DS>
 __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs a, ListWs w) {
     extern __shared__ __align__(16) char smem[];
     __shared__ uint32_t cnt, last;
     const uint32_t nf = *a.flag_count;
-    if (nf == 0) return;
+    if (nf == 0 || nf > SL_RESCUE_MAX) return;
     uint64_t* keys = reinterpret_cast<uint64_t*>(smem);
     const int tid = threadIdx.x, d = ix.d, M = ix.M, k = a.kout;
     float* r = reinterpret_cast<float*>(smem + SL_TOP * 8);  // [d]
     uint32_t* sl_l = reinterpret_cast<uint32_t*>(r + (d + 3) / 4 * 4);  // [P] lists, first positions, lengths
     uint32_t *sl_o = sl_l + a.P, *sl_n = sl_o + a.P;
-    const uint32_t S = nf >= gridDim.x ? 1u : min(64u, gridDim.x / nf);
+    // workgroups per query; their keys are merged in one sort
+    const uint32_t S = min(min(64u, SL_RESCUE / nf), max(8u, (SL_TOP - 2 * VGPU_BLOCK) / (uint32_t)k));
     for (uint32_t job = blockIdx.x; job < nf * S; job += gridDim.x) {
         const uint32_t f = job / S, sl = job % S, q = a.flag_list[f];
         const uint32_t* pr = a.probe + (size_t)q * a.P;
-        const uint64_t E = a.qstat[(size_t)q * QSTAT_WORDS];
+        const uint32_t kept = w.scount[q];
+        const bool all_kept = kept <= (uint32_t)w.cap;
+        const uint64_t E = all_kept ? kept : a.qstat[(size_t)q * QSTAT_WORDS];
         const uint64_t e0 = E * sl / S, e1 = E * (sl + 1) / S;
         __syncthreads();
         if (tid == 0) cnt = 0u;
@@ -1101,8 +1109,25 @@ __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs 
         }
         __syncthreads();
         SlTop top{keys, &cnt, ~0ull};
+        if (all_kept) {
+            const uint2* sv = w.surv + (size_t)q * w.cap;
+            for (uint64_t b = e0; b < e1; b += VGPU_BLOCK) {
+                const bool ok = b + tid < e1;
+                const uint32_t x = sv[ok ? b + tid : e0].x, slot = x >> w.tbits;
+                const size_t pos = (size_t)sl_o[slot] + (x & ((1u << w.tbits) - 1u));
+                const float* c = a.rres ? a.rres + ((size_t)q * a.P + slot) * d : ix.centroids + (size_t)sl_l[slot] * d;
+                float s = 0.0f;
+#pragma unroll 4
+                for (int m = 0; m < M; m++) {
+                    const float* cw = ix.codebooks + ((size_t)m * ix.K + ix.codes[pos * M + m]) * ix.ds;
+                    s = __fadd_rn(s, sl_sub<DS>(a.qn + (size_t)q * d + m * ix.ds, c + m * ix.ds, cw, ix.ds,
+                                                a.rres != nullptr));
+                }
+                sl_top_add(top, cand_key(s, ix.list_ids[pos]), ok, k);
+            }
+        }
         uint64_t at = 0;  // entries of the lists before
-        for (int p = 0; p < a.P && at < e1; p++) {
+        for (int p = 0; !all_kept && p < a.P && at < e1; p++) {
             const uint32_t l = sl_l[p], o0 = sl_o[p], len = sl_n[p];
             const uint64_t lo = at > e0 ? at : e0, hi = at + len < e1 ? at + len : e1;
             if (lo < hi) {
@@ -1126,26 +1151,24 @@ __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs 
             at += len;
         }
         uint32_t n = sl_top_end(top, k);
-        if (S > 1) {
-            uint64_t* part = w.rescue + (size_t)f * S * k;
-            for (int i = tid; i < k; i += VGPU_BLOCK) part[sl * k + i] = (uint32_t)i < n ? keys[i] : ~0ull;
-            __threadfence();
-            __syncthreads();
-            if (tid == 0) last = atomicAdd(&w.rescued[f], 1u) == S - 1u;
-            __syncthreads();
-            if (!last) continue;
-            __threadfence();
-            if (tid == 0) cnt = 0u;
-            top.thr = ~0ull;
-            __syncthreads();
-            for (uint32_t b = 0; b < S * (uint32_t)k; b += VGPU_BLOCK) {
-                const bool ok = b + tid < S * (uint32_t)k;
-                const uint64_t key =
-                    ok ? __hip_atomic_load(part + b + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~0ull;
-                sl_top_add(top, key, ok && key != ~0ull, k);
-            }
-            n = sl_top_end(top, k);
+        uint64_t* part = w.rescue + (size_t)f * S * k;
+        for (int i = tid; i < k; i += VGPU_BLOCK) part[sl * k + i] = (uint32_t)i < n ? keys[i] : ~0ull;
+        __threadfence();
+        __syncthreads();
+        if (tid == 0) last = atomicAdd(&w.rescued[f], 1u) == S - 1u;
+        __syncthreads();
+        if (!last) continue;
+        __threadfence();
+        if (tid == 0) cnt = 0u;
+        top.thr = ~0ull;
+        __syncthreads();
+        for (uint32_t b = 0; b < S * (uint32_t)k; b += VGPU_BLOCK) {
+            const bool ok = b + tid < S * (uint32_t)k;
+            const uint64_t key =
+                ok ? __hip_atomic_load(part + b + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~0ull;
+            sl_top_add(top, key, ok && key != ~0ull, k);
         }
+        n = sl_top_end(top, k);
         for (int j = tid; j < k; j += VGPU_BLOCK)
             scan_emit(a, (int)q, j, (uint32_t)j < n ? keys[j] : ~0ull, (uint32_t)j < n);
         __syncthreads();
@@ -1206,7 +1229,6 @@ static void launch_rescue(const DevIndex& ix, const ScanArgs& a, const ListWs& w
 void launch_list_pairs(const DevIndex& ix, const ScanArgs& a, ListWs& w, hipStream_t s) {
     w.qw = list_count_queries(a.nq);
     w.nwg = (a.nq + w.qw - 1) / w.qw;
-    launch_zero_words(reinterpret_cast<unsigned long long*>(w.heads), 2 + SL_RESCUE / 2, s);
     const size_t lds = (size_t)ix.L * 4;
     ensure_dyn_lds((const void*)list_count_kernel, lds);
     hipLaunchKernelGGL(list_count_kernel, dim3((a.nq + w.qw - 1) / w.qw), dim3(1024), lds, s, ix, a, w);
@@ -1235,6 +1257,11 @@ void launch_scan_list(const DevIndex& ix, const ScanArgs& a, const ListWs& ws, h
     if (a.kout <= 16) launch_final<64>(ix, a, w, s);
     else launch_final<256>(ix, a, w, s);
     launch_rescue(ix, a, w, s);
+    ScanArgs e = a;  // more flagged queries than that: the EXACT kernel
+    e.exact = 1;
+    e.only_flagged = 1;
+    e.flag_over = SL_RESCUE_MAX;
+    launch_scan8_exact(ix, e, s);
 }
 
 }  // namespace vgpu

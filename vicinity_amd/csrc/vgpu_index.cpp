@@ -918,7 +918,7 @@ size_t IvfpqIndex::ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) c
         carve(lw.cnt, (size_t)SL_COUNT_WG * L);
         carve(lw.first, (size_t)SL_COUNT_WG * L);
         carve(lw.first1, (size_t)SL_COUNT_WG * L);
-        carve(lw.heads, 4 + SL_RESCUE);
+        carve(lw.heads, 4 + SL_RESCUE_MAX);
         lw.rescued = lw.heads + 4;
         carve(lw.rescue, SL_RESCUE * pl.kout);
         lw.ld = lshape.contig ? (int)d : lshape.KT * 32;

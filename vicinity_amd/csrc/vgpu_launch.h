@@ -59,7 +59,8 @@ struct ScanArgs {
     int kout = 0;                   // results kept per query (k, or the rerank pool)
     int kk = 0;                     // FAST: entries a flush keeps (> kout); EXACT: kout
     int exact = 0;                  // 1 = EXACT mode
-    int only_flagged = 0;           // EXACT: run the queries of flag_list only
+    int only_flagged = 0;           // EXACT: run the queries of flag_list only,
+    int flag_over = 0;              // when there are more of them than this
     uint32_t* flag_list = nullptr;  // [nq] queries FAST could not prove (appended by FAST)
     uint32_t* flag_count = nullptr; // entries of flag_list (zeroed by launch_finish)
     uint32_t* out_vidx = nullptr;   // [nq*kout] insertion indices, 0xffffffff padding
@@ -190,7 +191,8 @@ inline int list_count_queries(int nq) {
     const int q = (nq + SL_COUNT_WG - 1) / SL_COUNT_WG;
     return q < 16 ? 16 : q;
 }
-#define SL_RESCUE 512       // workgroups of the flagged queries' exhaustive scan
+#define SL_RESCUE 512u      // workgroups of list_rescue_kernel
+#define SL_RESCUE_MAX 64u   // flagged queries it takes (more: the EXACT kernel)
 #define SL_MAX_LISTS 32768  // the pair count's LDS
 // Device workspace of one chunk (sizes in ws_layout).
 struct ListWs {
@@ -210,7 +212,7 @@ struct ListWs {
     float* padded = nullptr;      // [nq ld] the queries' padded copy, filled by the pair count
     uint32_t* cnt = nullptr;      // [nwg L] pairs (low half) and sample pairs (high half) of each list
     uint32_t *first = nullptr, *first1 = nullptr;  // [nwg L] first pair, first sample pair
-    uint32_t* heads = nullptr;    // [4] sample pairs, sample items, pairs, items; zeroed with rescued
+    uint32_t* heads = nullptr;    // [4] sample pairs, sample items, pairs, items; rescued follows
     uint32_t* pos = nullptr;      // [nq P] place in the (workgroup, list)'s pairs, in its sample pairs
     uint32_t* tbase = nullptr;    // [nq P] sample tiles of the query's nearer lists
     uint32_t *pairs = nullptr, *pairs1 = nullptr;  // [nq P] pair words by list
@@ -220,7 +222,7 @@ struct ListWs {
     float* bound = nullptr;       // [nq]
     float* gbound = nullptr;      // [nq 16 tcap] upper bounds of the sample's distances
     uint2* surv = nullptr;        // [nq cap] (label, distance bits)
-    uint32_t* rescued = nullptr;  // [SL_RESCUE] finished workgroups of each flagged query
+    uint32_t* rescued = nullptr;  // [SL_RESCUE_MAX] finished workgroups of each flagged query
     uint64_t* rescue = nullptr;   // [SL_RESCUE kout] their keys
 };
 // Work items of a chunk of nq queries, at most: blocks of ipairs pairs x 16 segments.
