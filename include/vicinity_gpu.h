@@ -327,6 +327,13 @@ int vgpu_test_bound_list(size_t padded_d, size_t M, size_t ds, float t0, float y
 /* Which scan a batch search of nq queries takes now: 0 the mode's own, 1 the
  * scan by inverted list (a test hook; no device call). */
 int vgpu_test_scan_route(vgpu_ivfpq *h, size_t nq, size_t k, size_t nprobe, size_t rerank_pool, int *out);
+/* The rule behind it for an index of n entries in L lists: sample tiles per
+ * query of the scan by inverted list, 0 the mode's own scan. */
+int vgpu_test_list_rule(size_t d, size_t M, size_t K, size_t L, size_t n, size_t nq, size_t P, size_t k, int opq,
+                        int *out);
+/* always != 0: every batch search whose shape has the scan by inverted list
+ * takes it, also where the rule prefers the mode's own scan. */
+int vgpu_test_set_list_scan(vgpu_ivfpq *h, int always);
 int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float *out_bf16x3, float *out_fp32);
 /* ib -1: the flat score's bound before packing (k above 32). */
 int vgpu_test_bound_flat(size_t d, int metric, float qn, float xn, int ib, float *out);

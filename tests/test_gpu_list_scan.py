@@ -25,6 +25,14 @@ def _route(ix, nq, k, nprobe, pool=0):
     return out.value
 
 
+def _always(ix, on=1):
+    """The scan by list for every batch whose shape has it: these small indexes
+    are for its edges, not for where it is the faster scan (test_rule)."""
+    from vicinity_amd import _lib
+
+    _lib.check(_lib.load().vgpu_test_set_list_scan(ix._h, on))
+
+
 def _index(oracle, rng, n, d, L, M, K, rotation=None, x=None, together=None):
     """(GPU index, oracle index) over mixture data; the lists are cut from a
     random assignment with ragged sizes, one empty and one of three entries
@@ -58,6 +66,7 @@ def _index(oracle, rng, n, d, L, M, K, rotation=None, x=None, together=None):
     ix = v.IVFPQIndex(d, num_clusters=L, num_codebooks=M, codebook_size=K, nprobe=4,
                       use_opq=rotation is not None)
     ix.load_artifacts(cent, books, off, order, codes, vectors=x, rotation=rotation)
+    _always(ix)
     oix = oracle.Index(cent, books.reshape(-1), off, order, codes, np.arange(n, dtype=np.uint32), x, M, K,
                        rotation)
     return ix, oix, x
@@ -115,6 +124,77 @@ def test_equal_distances_beyond_the_buffers(oracle, copies, k):
     q = (q + 1e-3 * rng.standard_normal(q.shape)).astype(np.float32)
     _same(ix, oix, q, k, 16)
     assert ix.last_stats()["fallback_queries"] >= 40
+
+
+def _rule(d, M, K, L, n, nq, P, k, opq=0):
+    from vicinity_amd import _lib
+
+    out = ctypes.c_int(-1)
+    _lib.check(_lib.load().vgpu_test_list_rule(d, M, K, L, n, nq, P, k, opq, ctypes.byref(out)))
+    return out.value
+
+
+@pytest.mark.parametrize("d,M,K,L,n,nq,P,k,opq", [
+    # the sample's bound leaves more survivors than a buffer holds: few long lists, a large k
+    (128, 16, 256, 256, 1_000_000, 1000, 64, 100, 0), (128, 16, 256, 16, 300_000, 1000, 8, 100, 0),
+    (128, 16, 256, 1, 300_000, 500, 1, 10, 0), (128, 16, 256, 2, 300_000, 500, 2, 10, 0),
+    (128, 16, 256, 64, 300_000, 1000, 64, 100, 0), (128, 16, 256, 16, 300_000, 5000, 8, 100, 1),
+    (100, 50, 16, 1, 300_000, 500, 1, 100, 0), (100, 50, 16, 8, 300_000, 500, 4, 100, 0),
+    # rescoring by odd widths costs more than the lookups saved
+    (96, 16, 256, 1024, 300_000, 10_000, 32, 100, 0), (96, 32, 256, 1024, 300_000, 10_000, 32, 200, 0),
+    (96, 6, 256, 1024, 300_000, 10_000, 32, 100, 0), (128, 4, 256, 1024, 300_000, 10_000, 32, 100, 0),
+    # small codebooks: cheap tables and lookups
+    (96, 8, 32, 1024, 300_000, 1200, 32, 10, 0), (96, 4, 64, 1024, 300_000, 2500, 32, 10, 0),
+    (96, 16, 64, 1024, 300_000, 600, 32, 10, 0),
+])
+def test_rule_keeps_the_other_scan_where_it_is_faster(d, M, K, L, n, nq, P, k, opq):
+    assert _rule(d, M, K, L, n, nq, P, k, opq) == 0
+
+
+@pytest.mark.parametrize("d,M,K,L,n,nq,P,k,opq,tiles", [
+    (128, 16, 256, 4096, 1_000_000, 10_000, 32, 100, 0, 32), (25, 25, 256, 1024, 1_183_514, 10_000, 32, 10, 0, 32),
+    (96, 48, 256, 16_384, 10_000_000, 10_000, 64, 10, 0, 32), (128, 16, 256, 2048, 500_000, 5000, 32, 100, 1, 32),
+    (100, 50, 16, 2048, 1_000_000, 10_000, 64, 100, 0, 128), (100, 50, 16, 64, 300_000, 500, 64, 100, 0, 128),
+    # longer lists: a larger sample
+    (100, 25, 256, 64, 300_000, 500, 16, 10, 0, 64), (100, 25, 256, 64, 300_000, 500, 64, 10, 0, 256),
+    (100, 25, 256, 128, 300_000, 3000, 4, 100, 0, 64), (128, 16, 256, 512, 1_000_000, 1000, 32, 100, 0, 256),
+])
+def test_rule_takes_the_scan_by_list(d, M, K, L, n, nq, P, k, opq, tiles):
+    assert _rule(d, M, K, L, n, nq, P, k, opq) == tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,tiles", [(9000, 64), (25_000, 128), (50_000, 256)])
+def test_larger_samples(oracle, n, tiles):
+    _print_case(f"list scan: samples of {tiles} tiles")
+    rng = np.random.default_rng(n)
+    x = rng.random((n, 25)).astype(np.float32)
+    ix, oix, _ = _index(oracle, rng, n, 25, 6, 25, 256, x=x)
+    q = rng.random((1501, 25)).astype(np.float32)
+    assert _rule(25, 25, 256, 6, n, len(q), 6, 100) == tiles
+    _same(ix, oix, q, 100, 6)
+    assert ix.last_stats()["fallback_queries"] < 15
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opq", [False, True])
+def test_unclustered_rows_in_few_long_lists(oracle, opq):
+    """Uniform rows, two lists, k 100: with the scan by list nearly every query
+    left more survivors than its buffer holds.  The mode's own scan is taken,
+    and the scan by list still agrees."""
+    _print_case(f"list scan: uniform rows in two lists, opq {opq}")
+    rng = np.random.default_rng(8)
+    n, d = 40_000, 32
+    x = rng.random((n, d)).astype(np.float32)
+    rot = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((d, d)))[0].astype(np.float32)) if opq else None
+    ix, oix, _ = _index(oracle, rng, n, d, 6, 8, 256, rotation=rot, x=x)
+    q = rng.random((200, d)).astype(np.float32)
+    _same(ix, oix, q, 100, 6)
+    assert ix.last_stats()["fallback_queries"] > 64  # more than list_rescue_kernel takes
+    _same(ix, oix, q[:20], 100, 6)
+    assert 0 < ix.last_stats()["fallback_queries"] <= 64
+    _always(ix, 0)
+    _same(ix, oix, q, 100, 6, route=0)
 
 
 @pytest.mark.gpu

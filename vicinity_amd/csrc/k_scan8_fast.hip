@@ -1819,22 +1819,18 @@ static int table_copies(const DevIndex& ix) {
     return ix.tcodes && scan8_fast_blocks_supported(ix.M, ix.K, ix.ds) ? 1 : 0;
 }
 
-// Static table bytes of the specialisations (compile-time M, K = 256).
-static size_t static_lut_bytes(const DevIndex& ix) {
-    if (ix.K != 256) return 0;
-    const int nc = table_copies(ix);
-    switch (ix.M) {
-        case 4: case 8: case 16: case 32: case 48: case 64: case 96:
-            return (size_t)ix.M * 256 * 4 * (nc ? nc : 1);
-        default: return 0;
-    }
+// The codebook counts launch_scan8_fast fixes at compile time, with 256
+// codewords: rows of whole 16-byte or 4-byte loads that index files commonly
+// have.  Any other count takes the
+// run-time kernel, whose rows are read a byte at a time.
+bool scan8_fast_compiled(int M, int K) {
+    return K == 256 && (M == 4 || M == 8 || M == 16 || M == 32 || M == 48 || M == 64 || M == 96);
 }
 
-// The codebook counts and subvector widths launch_scan8_fast fixes at compile time.
-bool scan8_fast_compiled(int M, int K, int ds) {
-    if (K != 256) return false;
-    const bool m = M == 4 || M == 8 || M == 16 || M == 32 || M == 48 || M == 64;
-    return m && (ds == 2 || ds == 3 || ds == 4 || ds == 6 || ds == 8 || ds == 12 || ds == 16);
+// Static table bytes of the specialisations (compile-time M, K = 256).
+static size_t static_lut_bytes(const DevIndex& ix) {
+    const int nc = table_copies(ix);
+    return scan8_fast_compiled(ix.M, ix.K) ? (size_t)ix.M * 256 * 4 * (nc ? nc : 1) : 0;
 }
 
 size_t scan8_fast_lds_bytes(const DevIndex& ix, const ScanArgs& a) {

@@ -1242,6 +1242,7 @@ void launch_list_bound(const ScanArgs& a, const ListWs& w, hipStream_t s) {
     switch (w.tcap) {
         case 32: hipLaunchKernelGGL(list_bound_kernel<2>, bg, dim3(256), 0, s, a, w); break;
         case 64: hipLaunchKernelGGL(list_bound_kernel<4>, bg, dim3(256), 0, s, a, w); break;
+        case 256: hipLaunchKernelGGL(list_bound_kernel<16>, bg, dim3(256), 0, s, a, w); break;
         default: hipLaunchKernelGGL(list_bound_kernel<8>, bg, dim3(256), 0, s, a, w); break;
     }
 }

@@ -644,6 +644,22 @@ int vgpu_test_scan_route(vgpu_ivfpq* h, size_t nq, size_t k, size_t nprobe, size
     });
 }
 
+int vgpu_test_list_rule(size_t d, size_t M, size_t K, size_t L, size_t n, size_t nq, size_t P, size_t k, int opq,
+                        int* out) {
+    return guard([&] {
+        need(out && d && M && d % M == 0 && L, VGPU_ERR_INVALID_PARAMETER, "bad argument");
+        *out = vgpu::list_scan_tiles(d, M, K, d / M, L, n, nq, P, k, opq != 0);
+    });
+}
+
+int vgpu_test_set_list_scan(vgpu_ivfpq* h, int always) {
+    return guard([&] {
+        need(h, VGPU_ERR_INVALID_PARAMETER, "null handle");
+        std::unique_lock<std::shared_mutex> lk(h->ix->mu);
+        h->ix->list_always = always != 0;
+    });
+}
+
 int vgpu_test_bound_coarse(size_t d, float qn, float cmax, float* out_bf16x3, float* out_fp32) {
     return guard([&] {
         need(out_bf16x3 && out_fp32 && d, VGPU_ERR_INVALID_PARAMETER, "bad argument");

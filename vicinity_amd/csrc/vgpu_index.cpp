@@ -766,18 +766,80 @@ vgpu_search_stats IvfpqIndex::last_stats() {
     return stats;
 }
 
+// Sample tiles (per query) of the scan by inverted list for nq queries of P
+// probes into n entries, or 0 where the mode's own scan is the better one.
+//
+// Survivors.  The sample is S = 16 tiles of the query's E entries, and the
+// k-th smallest of it bounds the query's k-th distance, so k E / S entries are
+// within the bound on average and, where the sample is no better than a random
+// one, (k + 3.1 sqrt(k) + 3) E / S in one query of a thousand (the sum of k
+// exponentials).  The sample grows until that is half a survivor buffer; a
+// search whose largest sample leaves more than 0.85 of one keeps the other
+// scan, since every entry of a query that overflows is scored a second time.
+// Without this, 1000 queries, k 100: 1M uniform x 128, 512 lists, 32 probes
+// 443 -> 6086 us; 300k x 128, 16 lists, 8 probes 512 -> 6492.  A 4-bit query
+// that overflows is only scanned again by fastscan_kernel, and the sample is
+// of the nearest lists, so there 16 lists are counted: 300k x 100, M 50, k 100,
+// 500 queries, 1 list 2706 -> 5109 us, 8 lists and 4 probes 734 -> 1119; 64
+// lists and 64 probes 888 -> 382, uniform rows 1946 -> 1895.
+int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n, size_t nq, size_t P, size_t kout,
+                    bool opq) {
+    const double k = (double)kout, pairs = (double)nq * P, len = (double)n / L, entries = pairs * len;
+    auto survivors = [&](double probes, int tiles) {
+        return (k + 3.1 * std::sqrt(k) + 3.0) * probes * len / (16.0 * tiles);
+    };
+    if (K == 16) {
+        // Cost.  The 4-bit scan by list has about 120 us of launches and sampling
+        // above fastscan_kernel's and less per entry; both build a table per
+        // pair, so lists must be long enough for the entries to matter, less so
+        // at a large k, which slows fastscan_kernel's wave buffers.  Whole
+        // search, fastscan -> by list, k 10 / k 100 at 31M / 26M entries: M 16,
+        // 390 per list, 250 -> 220 / 322 -> 251 us; M 25, 586 per list, 322 ->
+        // 224 / 340 -> 239; M 50, 488 per list, 432 -> 335 / 476 -> 364; M 64, 293
+        // per list, 547 -> 404 / 626 -> 406; M 50, 136 per list, k 100, 752 -> 555.
+        const bool large_k = kout >= 64;
+        if (pairs < 16.0 * L || entries < (large_k ? 25e6 : 30e6) || n < (large_k ? 96 : 256) * L) return 0;
+        return survivors(std::min<double>(P, 16), 128) <= SL_CAP16 ? 128 : 0;
+    }
+    // up to three codebooks: the entries of a long list share codes, and the ties
+    // overflow the buffers (300k x 32, 128 lists, 1000 queries 221 -> 426 us)
+    if (pairs < 1.5 * L || (opq && M < 4 && len > 512)) return 0;
+    int tiles = kout <= 128 ? 32 : 64;
+    while (tiles < 256 && survivors(P, tiles) > 0.5 * SL_CAP) tiles *= 2;
+    if (survivors(P, tiles) > 0.85 * SL_CAP) return 0;
+    // Cost, in ns (entries in ps), as measured at 300k rows in 1024 lists (32 probes), 4096 (64)
+    // and 128 (4) over 43 shapes.  An entry of the scan by list costs its
+    // matrix product, one of the other scans M lookups, with the codebook count
+    // compiled in or not.  A result costs its rescoring, whose
+    // codewords are gathered whole where the width is 4 or 8 and float by float
+    // elsewhere; the other scans have part of it too.  The EXACT scan of an OPQ
+    // index builds a table per pair.  The scan by list has more launches, a
+    // sample, and arrays over the lists; few wide codebooks, whose code several
+    // virtual codebooks share, gather the same rows of the table at once.
+    // Before, entries times codebooks alone decided: 10,000 queries, 94M
+    // entries, 16 codebooks of 6, k 100 445 -> 810 us; 32 of 3, k 200 927 ->
+    // 1246; 1200 queries, 8 codebooks of 32 codewords of 12 120 -> 170.
+    const ListShape sh = list_shape((int)d, (int)M, (int)K, (int)ds);
+    const bool compiled = scan8_fast_compiled((int)M, (int)K);
+    const double m = (double)M, dd = (double)d;
+    const double by_code = compiled ? 1.0 + 0.17 * m : K == 256 ? 2.6 + 0.24 * m : 2.2 + 0.19 * m;
+    const double rescore = ds == 8   ? 0.04 + 0.0006 * dd
+                           : ds == 4 ? 0.07 + 0.0015 * dd
+                           : ds <= 2 ? (M > 32 && M < 64 ? 0.0075 : 0.0105) * m
+                           : ds < 8  ? 0.06 + 0.005 * dd
+                                     : 0.05 + 0.0085 * dd;
+    const double tables =
+        opq ? pairs * (compiled ? 0.03 * dd * (double)K / 256.0 + 0.05 * m - 0.5 : 20.0) : 0.0;
+    const double fixed = (opq ? 16e3 : (compiled ? 45e3 : 35e3) + 14e3 * (sh.parts - 1)) + 2.5 * (double)L;
+    // a wave walks a sixteenth of a list, at least: 300k rows in one list, 500
+    // queries, k 1 594 -> 994 us
+    const double by_list = std::max(1e-3 * entries * (0.6 + 0.25 * sh.KT), 4.5 * len);
+    const double saved = 1e-3 * entries * by_code + tables - by_list;
+    return saved > fixed + (double)nq * k * (rescore - 0.0025 * (compiled || opq ? m : dd)) ? tiles : 0;
+}
+
 // Whether a search of nq queries takes the scan by inverted list, and its
-// buffer sizes.  Its fixed cost is about 40 us of launches above the FAST
-// scan's; per million scanned entries it costs 0.7 us (25 dimensions) to 1.6
-// us (128), where the FAST scan's lookups cost about 2.2 us at 8 codebooks, 3
-// at 16 and 9 at 48 (15 to 20 where the codebook count or the subvector width is
-// not one it is compiled for, and the EXACT scan of an OPQ index 22), and a
-// large k narrows the gap (its rescoring is the same).  Measured, FAST -> by
-// list: 1M x 128, M 16, k 10, 15M entries 149 -> 151 us, 39M 225 -> 180; k 100,
-// 39M 303 -> 314, 68M 461 -> 454; 300k x 32, M 8, 19M 113 -> 121, 76M 235 ->
-// 170; 1M x 96, M 48, 8M 166 -> 147; 1M x 100, M 25, 4M 203 -> 136; OPQ 500k x
-// 128, 0.8M 166 -> 154, 8M 309 -> 202.  A few wide codebooks cost few lookups
-// and many products: 300k x 96, M 8, 38M 208 -> 285.
+// buffer sizes.
 static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
     if (!ix.lshape.ok || (ix.K != 16 && ix.mode != VGPU_MODE_FAST) || pl.wide || pl.P == 0 || pl.kout > 256 || ix.L > SL_MAX_LISTS ||
         (pl.opq && !ix.lshape.contig))
@@ -786,36 +848,10 @@ static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
     while (((size_t)1 << sb) < pl.P) sb++;
     pl.tbits = std::min(26, 32 - sb);
     if (ix.max_list >= (1u << pl.tbits)) return false;
-    const double pairs = (double)nq * pl.P, lookups = pairs * ix.n() / ix.L * ix.M;
-    if (ix.K == 16) {
-        // The 4-bit scan by list costs about 120 us of launches and sampling
-        // above fastscan_kernel's and less per entry; both build a table per
-        // pair, so lists must be long enough for the entries to matter, less so
-        // at a large k, which slows fastscan_kernel's wave buffers.  Whole
-        // search, fastscan -> by list, k 10 / k 100: M 50, 488 per list, 9M
-        // entries 341 -> 310 / 413 -> 333 us, 31M 446 -> 400 / 518 -> 448, 313M
-        // 2292 -> 1054 / 2615 -> 1153; M 25, 586 per list, 28M 281 -> 318 / 394 ->
-        // 361, 94M 677 -> 464 / 1031 -> 535; M 16, 390 per list, 9M 157 -> 231 /
-        // 245 -> 256, 31M 347 -> 275 / 614 -> 309; M 50, 195 per list, 31M 589 ->
-        // 662 / 827 -> 667; M 64, 122 per list, 12M 424 -> 465 / 550 -> 499, 39M
-        // 1055 -> 984 / 1361 -> 1001.
-        const double entries = pairs * ix.n() / ix.L;
-        const bool large_k = pl.kout >= 64;
-        if (pairs < 16.0 * ix.L || entries < (large_k ? 25e6 : 30e6) || ix.n() < (large_k ? 96 : 256) * ix.L) return false;
-        pl.tcap = 128;
-        pl.cap = 6144;
-        return true;
-    }
-    if (pairs < 1.5 * ix.L) return false;
-    if (pl.opq) {
-        if (lookups < 0.02e9) return false;
-    } else if (!scan8_fast_compiled((int)ix.M, (int)ix.K, (int)ix.ds)) {
-        if (lookups < 0.08e9) return false;
-    } else if (lookups < 0.35e9 + 0.005e9 * (double)pl.kout || 10 * ix.M < (size_t)ix.lshape.KT * 32) {
-        return false;
-    }
-    pl.tcap = pl.kout <= 128 ? 32 : 64;
-    pl.cap = 4096;
+    pl.tcap = list_scan_tiles(ix.d, ix.M, ix.K, ix.ds, ix.L, ix.n(), nq, pl.P, pl.kout, pl.opq);
+    if (!pl.tcap && ix.list_always) pl.tcap = ix.K == 16 ? 128 : pl.kout <= 128 ? 32 : 64;
+    if (!pl.tcap) return false;
+    pl.cap = ix.K == 16 ? SL_CAP16 : SL_CAP;
     pl.rcap = 256;
     while ((size_t)pl.rcap < 4 * pl.kout) pl.rcap <<= 1;
     return true;

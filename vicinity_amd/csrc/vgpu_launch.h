@@ -194,10 +194,12 @@ inline int list_count_queries(int nq) {
 #define SL_RESCUE 512u      // workgroups of list_rescue_kernel
 #define SL_RESCUE_MAX 64u   // flagged queries it takes (more: the EXACT kernel)
 #define SL_MAX_LISTS 32768  // the pair count's LDS
+#define SL_CAP 4096         // survivors a query's buffer holds
+#define SL_CAP16 6144       // the same for 4-bit codes
 // Device workspace of one chunk (sizes in ws_layout).
 struct ListWs {
     ListShape sh;
-    int tcap = 0;   // sample tiles per query: 32, 64 or 128
+    int tcap = 0;   // sample tiles per query: 32, 64, 128 or 256
     int seg = 16;   // entry tiles (16 entries each) per work item, at least
     int ipairs = 64;  // pairs per work item, at most (a multiple of 16)
     int cap = 0;    // survivors per query
@@ -314,8 +316,8 @@ void launch_bias(const DevIndex& ix, float* bias, hipStream_t s);
 #define TBLK_BYTES(M) (16 * (size_t)(M) + 64)
 // Whether the FAST scan reads transposed blocks for this shape.
 bool scan8_fast_blocks_supported(int M, int K, int ds);
-// Whether the FAST scan has this codebook count and width at compile time.
-bool scan8_fast_compiled(int M, int K, int ds);
+// Whether the FAST scan has this codebook count at compile time.
+bool scan8_fast_compiled(int M, int K);
 // The FAST scan shapes whose per-query tables come from launch_t2_tables
 // (16 codebooks of 256 codewords on transposed blocks, ds 2, 4 or 8).
 bool scan8_fast_uses_tables(const DevIndex& ix);

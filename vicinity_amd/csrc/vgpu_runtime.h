@@ -70,6 +70,11 @@ struct DevBuf {
     }
 };
 
+// The rule by which a search takes the scan by inverted list (its sample
+// tiles per query; 0: the mode's own scan).
+int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n, size_t nq, size_t P, size_t kout,
+                    bool opq);
+
 // Sizes of one search call's device workspace: per query chunk, the
 // normalised queries, coarse candidates or score rows, probe lists, scan
 // results and statistics rows, plus the per-call scalars.
@@ -253,6 +258,7 @@ struct IvfpqIndex {
     // Filtered search under OPQ rotates at most this many floats of residuals
     // per pass (queries go in chunks); settable for tests.
     size_t rres_limit = (size_t)1 << 28;
+    bool list_always = false;  // a test hook: the scan by inverted list wherever the shape has it
 
   private:
     // Every chunk of one search: coarse, select, scan, rerank and finish.
