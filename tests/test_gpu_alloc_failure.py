@@ -110,3 +110,38 @@ def test_flat_add_recovers_from_allocation_failure(oracle, fail):
     ids, dists = fx.search(q, 10)
     oids, odists = oracle.flat_search(base, q, 10, metric=0)
     assert np.array_equal(ids, oids) and dists.tobytes() == odists.tobytes()
+
+
+@pytest.mark.parametrize("d,M,K", [(64, 16, 256), (50, 25, 256), (32, 16, 16)])
+def test_upload_without_memory_for_the_scan_by_list(oracle, fail, d, M, K):
+    """The list-scan arrays are optional: an upload that cannot hold them
+    succeeds, and a large batch takes the scan it has without them."""
+    from test_gpu_list_scan import _always, _index, _route
+
+    import vicinity_amd as v
+    from vicinity_amd import VicinityGpuError
+
+    _print_case(f"alloc failure: list-scan arrays, d={d} M={M} ksub={K}")
+    rng = np.random.default_rng(d)
+    ix, oix, x = _index(oracle, rng, 3000, d, 16, M, K)
+    art = ix.export()
+    q = (x[rng.integers(0, 3000, 500)] + 0.1 * rng.standard_normal((500, d))).astype(np.float32)
+    want = oix.search_batch(q, 10, 16)
+    without = 0
+    for after in range(40):
+        one = v.IVFPQIndex(d, num_clusters=16, num_codebooks=M, codebook_size=K, nprobe=16)
+        fail(after)
+        try:
+            one.load_artifacts(*(art[n] for n in ("centroids", "codebooks", "list_offsets", "list_ids", "codes")))
+        except VicinityGpuError:
+            continue
+        finally:
+            fail(0, 0)
+        _always(one)
+        route = _route(one, 500, 10, 16)
+        ids, dists = one.batch_search(q, 10)
+        assert np.array_equal(ids, want[0]) and dists.tobytes() == want[1].tobytes(), after
+        if route == 1:
+            break
+        without += 1
+    assert route == 1 and without >= 2

@@ -607,18 +607,24 @@ static uint32_t host_bf16(float x) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
+// Device memory that stays free beside the optional arrays of the scan by list:
+// a search's workspace takes up to 2.5 GiB (score rows, rotated residuals).
+static constexpr size_t kListHeadroom = (size_t)4 << 30;
+
 // Tiles, codeword table and dimension map of the scan by inverted list
 // (k_scan_list.hip).  Codewords or centroids that are not finite, or so large
-// that squared norms could overflow, leave the index without it.
+// that squared norms could overflow, leave the index without it, and so does
+// an index whose searches can never take it, or too little device memory.
 void IvfpqIndex::upload_list_scan() {
     lshape = list_shape((int)d, (int)M, (int)K, (int)ds);
     if (K == 16) {  // the 4-bit scan by list (k_fast_list.hip): nibbles, no table
         lshape.LW = fast_list_words((int)M);
         lshape.contig = true;
-        lshape.ok = fast_list_shape((int)M, (int)ds);
+        lshape.ok = fast_list_shape((int)M, (int)ds) && n() >= 96 * L;
     }
     max_list = 0;
     for (size_t l = 0; l < L; l++) max_list = std::max<uint32_t>(max_list, (uint32_t)(offsets[l + 1] - offsets[l]));
+    if (L > SL_MAX_LISTS || max_list >= (1u << 26) || (!rotation.empty() && !lshape.contig)) lshape.ok = false;
     // the score kernel's buffer loads take 32-bit byte offsets
     uint64_t tiles = 0;
     for (size_t l = 0; l < L; l++) tiles += (offsets[l + 1] - offsets[l] + 15) / 16;
@@ -626,25 +632,47 @@ void IvfpqIndex::upload_list_scan() {
     if (!(dix.cmax < 1e15f) || !(dix.rmax < 1e15f)) lshape.ok = false;
     for (float x : centroids) lshape.ok = lshape.ok && std::isfinite(x);
     for (float x : codebooks) lshape.ok = lshape.ok && std::isfinite(x);
-    if (!lshape.ok) {
-        d_lcodes.release();
-        d_ltable.release();
-        d_ltoff.release();
-        d_lbias.release();
-        d_lcent.release();
-        d_dimmap.release();
-        return;
+    if (lshape.ok) {
+        try {
+            upload_list_arrays();
+            size_t free = 0, total = 0;
+            VGPU_HIP(hipMemGetInfo(&free, &total));
+            lshape.ok = free >= kListHeadroom;
+        } catch (const Error& e) {
+            if (e.code != VGPU_ERR_OUT_OF_MEMORY) throw;
+            lshape.ok = false;  // every search has the scan it had without it
+        }
     }
+    if (lshape.ok) return;
+    d_lcodes.release();
+    d_ltable.release();
+    d_ltoff.release();
+    d_lbias.release();
+    d_lcent.release();
+    d_dimmap.release();
+    dix.lcodes = nullptr;
+    dix.lbias = nullptr;
+    dix.ltable = nullptr;
+    dix.ltoff = nullptr;
+    dix.ltiles = 0;
+}
+
+void IvfpqIndex::upload_list_arrays() {
+    // the copies from the host arrays below, also when an allocation throws
+    struct Wait {
+        hipStream_t s;
+        ~Wait() { (void)hipStreamSynchronize(s); }
+    };
     if (K == 16) {
         std::vector<uint32_t> off(L + 1, 0);
         for (size_t l = 0; l < L; l++) off[l + 1] = off[l] + (uint32_t)((offsets[l + 1] - offsets[l] + 15) / 16);
+        const Wait wait{stream};
         d_ltoff.upload(off.data(), L + 1, stream);
         d_lcodes.reserve((size_t)off[L] * 64 * lshape.LW);
         dix.ltoff = d_ltoff.p;
         dix.ltiles = off[L];
         dix.lcodes = d_lcodes.p;
         launch_fast_list_tiles(dix, d_lcodes.p, stream);
-        VGPU_HIP(hipStreamSynchronize(stream));  // before the host array goes
         return;
     }
     const int dsp = lshape.dsp, parts = lshape.parts, Mt = lshape.KT * 32 / dsp;
@@ -674,12 +702,13 @@ void IvfpqIndex::upload_list_scan() {
     std::vector<double> cwn(M * K, 0.0);
     for (size_t i = 0; i < M * K; i++)
         for (size_t j = 0; j < ds; j++) cwn[i] += (double)codebooks[i * ds + j] * codebooks[i * ds + j];
+    std::vector<float> pc;  // centroids in padded order
     DevBuf<double> d_cwn;
+    const Wait wait{stream};
     d_cwn.upload(cwn.data(), cwn.size(), stream);
     d_ltoff.upload(toff.data(), L + 1, stream);
     d_ltable.upload(table.data(), table.size(), stream);
     d_dimmap.upload(map.data(), map.size(), stream);
-    std::vector<float> pc;  // centroids in padded order
     if (!lshape.contig) {
         const size_t ld = map.size();
         pc.assign(L * ld, 0.0f);
@@ -698,7 +727,6 @@ void IvfpqIndex::upload_list_scan() {
     dix.lcodes = d_lcodes.p;
     dix.lbias = d_lbias.p;
     launch_list_tiles(dix, d_cwn.p, lshape, d_lcodes.p, d_lbias.p, stream);
-    VGPU_HIP(hipStreamSynchronize(stream));  // before d_cwn and the host arrays go
 }
 
 static int fast_keep(size_t kout) {
@@ -841,9 +869,7 @@ int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n,
 // Whether a search of nq queries takes the scan by inverted list, and its
 // buffer sizes.
 static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
-    if (!ix.lshape.ok || (ix.K != 16 && ix.mode != VGPU_MODE_FAST) || pl.wide || pl.P == 0 || pl.kout > 256 || ix.L > SL_MAX_LISTS ||
-        (pl.opq && !ix.lshape.contig))
-        return false;
+    if (!ix.lshape.ok || (ix.K != 16 && ix.mode != VGPU_MODE_FAST) || pl.wide || pl.P == 0 || pl.kout > 256) return false;
     int sb = 0;
     while (((size_t)1 << sb) < pl.P) sb++;
     pl.tbits = std::min(26, 32 - sb);

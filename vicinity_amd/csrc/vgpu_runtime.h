@@ -286,7 +286,8 @@ struct IvfpqIndex {
     void rotate_slots(const float* d_qn, size_t nq, size_t P, const uint32_t* d_lists, float* out,
                       hipStream_t s);
     void snapshot_list_masks();
-    void upload_list_scan();  // the arrays of the scan by inverted list
+    void upload_list_scan();    // the arrays of the scan by inverted list, where it can be taken
+    void upload_list_arrays();
     void refresh_categories(hipStream_t s);
 };
 
