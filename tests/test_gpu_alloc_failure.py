@@ -145,3 +145,53 @@ def test_upload_without_memory_for_the_scan_by_list(oracle, fail, d, M, K):
             break
         without += 1
     assert route == 1 and without >= 2
+
+
+@pytest.mark.parametrize("d,M,K", [(64, 16, 256), (32, 16, 16)])
+def test_search_without_memory_for_the_scan_by_list(oracle, fail, d, M, K):
+    """A batch whose list-scan workspace cannot be had takes the scan it has
+    without it; the next batch takes the scan by list again."""
+    import torch
+
+    from test_gpu_list_scan import _index, _route
+    from vicinity_amd import VicinityGpuError
+
+    _print_case(f"alloc failure: list-scan workspace, d={d} M={M} ksub={K}")
+    rng = np.random.default_rng(d)
+    ix, oix, x = _index(oracle, rng, 3000, d, 16, M, K)
+    q = (x[rng.integers(0, 3000, 500)] + 0.1 * rng.standard_normal((500, d))).astype(np.float32)
+    want = oix.search_batch(q, 10, 16)
+    qd = torch.from_numpy(q).to("cuda:0")
+    assert _route(ix, 500, 10, 16) == 1
+
+    def search():
+        ids, dists = ix.search_batch_device(qd, 10, nprobe=16)
+        assert np.array_equal(ids.cpu().numpy(), want[0]) and dists.cpu().numpy().tobytes() == want[1].tobytes()
+        return ix.last_stats()["fast_appends"]  # the list scan: its survivors
+
+    fail(0, 4)  # both scans' workspaces, each twice
+    with pytest.raises(VicinityGpuError) as e:
+        ix.search_batch_device(qd, 10, nprobe=16)
+    _oom(e)
+    fail(0, 2)
+    without = search()
+    fail(0, 0)
+    assert search() != without
+    fail(0, 1)
+    ids, dists = ix.search_batch_device(qd, 10, nprobe=16)  # the workspace is there: nothing is allocated
+    assert np.array_equal(ids.cpu().numpy(), want[0])
+
+
+def test_search_tries_its_workspace_twice(fail):
+    """A failed workspace is tried again once the idle ones' memory is free."""
+    import vicinity_amd as v
+
+    w = v.datagen.ivfpq_small(n=6000, nq=1000)
+    _print_case("alloc failure: a larger workspace, once")
+    ix = v.IVFPQIndex(32, num_clusters=32, num_codebooks=8, codebook_size=256, nprobe=4, seed=3)
+    ix.add_items(w.base)
+    ix.build(kmeans_max_iter=3)
+    want = ix.batch_search(w.queries, 10)
+    fail(3)  # the queries, ids and distances are staged, then the workspace fails
+    ids, dists = ix.batch_search(np.concatenate([w.queries] * 3), 10)
+    assert np.array_equal(ids[:1000], want[0]) and dists[2000:].tobytes() == want[1].tobytes()

@@ -1003,6 +1003,40 @@ size_t IvfpqIndex::ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) c
     return (off + 255) & ~(size_t)255;
 }
 
+// Reserves the workspace of a call's plan and sets the pointers into it.
+// Before a call fails, the memory of idle workspaces is given back: each keeps
+// that of the largest call it served.
+WsPtrs IvfpqIndex::reserve_ws(SearchWs& ws, const SearchPlan& pl) {
+    const size_t bytes = ws_layout(pl, nullptr, nullptr);
+    try {
+        ws.arena.reserve(bytes);
+    } catch (const Error& e) {
+        if (e.code != VGPU_ERR_OUT_OF_MEMORY) throw;
+        {
+            std::lock_guard<std::mutex> lk(pool_mu);
+            for (auto& w : ws_pool) w->arena.release();
+        }
+        ws.arena.reserve(bytes);
+    }
+    WsPtrs w;
+    ws_layout(pl, ws.arena.p, &w);
+    return w;
+}
+
+// The same for a search.  The scan by list takes up to 0.8 GiB more than the
+// scans it replaces; where that cannot be had the search goes without it.
+WsPtrs IvfpqIndex::reserve_search_ws(SearchWs& ws, SearchPlan& pl, size_t nq, size_t nprobe) {
+    if (pl.list) {
+        try {
+            return reserve_ws(ws, pl);
+        } catch (const Error& e) {
+            if (e.code != VGPU_ERR_OUT_OF_MEMORY) throw;
+        }
+        pl = plan_search(nq, pl.k, nprobe, pl.pool);
+    }
+    return reserve_ws(ws, pl);
+}
+
 // Normalise (search.rs:55-62) and probe (search.rs:1602-1617) nq <= chunk
 // queries.  The fused path normalises in its prologue; P == 0 only normalises.
 void IvfpqIndex::coarse_probe(const float* d_q, size_t nq, size_t P, const SearchPlan& pl,
@@ -1249,14 +1283,11 @@ void IvfpqIndex::search_device(const float* d_q, size_t nq, size_t k, size_t npr
         stats = st;
         return;
     }
-    const SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
+    SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
     WsLease ws(*this, take_ws());
     if (!s) s = ws->stream;
     ws.used = s;
-    const size_t bytes = ws_layout(pl, nullptr, nullptr);
-    ws->arena.reserve(bytes);
-    WsPtrs w;
-    ws_layout(pl, ws->arena.p, &w);
+    const WsPtrs w = reserve_search_ws(*ws.ws, pl, nq, nprobe);
     run_search(d_q, nq, pl, w, d_ids, d_dists, s, ws.ws.get(), &st);
     std::lock_guard<std::mutex> lk(stats_mu);
     stats = st;
@@ -1355,15 +1386,13 @@ void IvfpqIndex::search_host(const float* q, size_t nq, size_t k, size_t nprobe,
         if (!std::isfinite(q[i])) throw Error(VGPU_ERR_INVALID_PARAMETER, "query contains a non-finite value");
     if (!built) throw Error(VGPU_ERR_NOT_BUILT, "IVF-PQ index: search before build");
     if (nq == 0 || k == 0) return;
-    const SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
+    SearchPlan pl = plan_search(nq, k, nprobe, pool, true);
     WsLease ws(*this, take_ws());
     hipStream_t s = ws->stream;
     ws->q.upload(q, nq * d, s);
     ws->ids.reserve(nq * k);
     ws->odist.reserve(nq * k);
-    ws->arena.reserve(ws_layout(pl, nullptr, nullptr));
-    WsPtrs w;
-    ws_layout(pl, ws->arena.p, &w);
+    const WsPtrs w = reserve_search_ws(*ws.ws, pl, nq, nprobe);
     vgpu_search_stats st{};
     st.nq = (uint32_t)nq;
     run_search(ws->q.p, nq, pl, w, ws->ids.p, ws->odist.p, s, ws.ws.get(), &st);
@@ -1389,9 +1418,7 @@ void IvfpqIndex::search_host_probed(const float* q, size_t nq, size_t P, const u
     else ws->gprobe.reserve(1);
     ws->ids.reserve(nq * k);
     ws->odist.reserve(nq * k);
-    ws->arena.reserve(ws_layout(pl, nullptr, nullptr));
-    WsPtrs w;
-    ws_layout(pl, ws->arena.p, &w);
+    const WsPtrs w = reserve_ws(*ws.ws, pl);
     vgpu_search_stats st{};
     st.nq = (uint32_t)nq;
     run_search(ws->q.p, nq, pl, w, ws->ids.p, ws->odist.p, s, ws.ws.get(), &st, ws->gprobe.p);
@@ -1410,9 +1437,7 @@ void IvfpqIndex::probe_host(const float* q, size_t nq, size_t nprobe, uint32_t* 
     WsLease ws(*this, take_ws());
     hipStream_t s = ws->stream;
     ws->q.upload(q, nq * d, s);
-    ws->arena.reserve(ws_layout(pl, nullptr, nullptr));
-    WsPtrs w;
-    ws_layout(pl, ws->arena.p, &w);
+    const WsPtrs w = reserve_ws(*ws.ws, pl);
     launch_zero_words(w.scal, kScalWords, s);
     uint32_t* cflag_count = reinterpret_cast<uint32_t*>(w.scal + kCFlagWord);
     for (size_t q0 = 0; q0 < nq; q0 += pl.chunk) {
@@ -1517,9 +1542,7 @@ void IvfpqIndex::search_filtered(const float* q, size_t nq, size_t k, const int*
     WsLease ws(*this, take_ws());
     hipStream_t s = ws->stream;
     ws->q.upload(q, nq * d, s);
-    ws->arena.reserve(ws_layout(pl, nullptr, nullptr));
-    WsPtrs w;
-    ws_layout(pl, ws->arena.p, &w);
+    const WsPtrs w = reserve_ws(*ws.ws, pl);
     ws->fqn.reserve(nq * d);
     std::vector<uint32_t> probes(nq * P);
     launch_zero_words(w.scal, kScalWords, s);

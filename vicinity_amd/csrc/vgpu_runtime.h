@@ -224,6 +224,9 @@ struct IvfpqIndex {
     SearchPlan plan_search(size_t nq, size_t k, size_t nprobe, size_t pool, bool by_list = false) const;
     // Bytes of a plan's workspace arena; with a base, also the pointers into it.
     size_t ws_layout(const SearchPlan& pl, uint8_t* base, WsPtrs* out) const;
+    // The plan's workspace; a search's plan may change where memory is short.
+    WsPtrs reserve_ws(SearchWs& ws, const SearchPlan& pl);
+    WsPtrs reserve_search_ws(SearchWs& ws, SearchPlan& pl, size_t nq, size_t nprobe);
     // Device-pointer batch search on stream s (null: the borrowed workspace's
     // stream); waits for completion.
     void search_device(const float* d_q, size_t nq, size_t k, size_t nprobe, size_t pool,
