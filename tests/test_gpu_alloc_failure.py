@@ -195,3 +195,29 @@ def test_search_tries_its_workspace_twice(fail):
     fail(3)  # the queries, ids and distances are staged, then the workspace fails
     ids, dists = ix.batch_search(np.concatenate([w.queries] * 3), 10)
     assert np.array_equal(ids[:1000], want[0]) and dists[2000:].tobytes() == want[1].tobytes()
+
+
+@pytest.mark.parametrize("d,k", [(48, 10), (48, 100), (160, 10)])
+def test_flat_without_memory_for_the_ranking_path(oracle, fail, d, k):
+    """The packed copy is optional, and a search whose buffer fails goes in
+    smaller passes."""
+    from vicinity_amd import FlatIndex
+
+    _print_case(f"alloc failure: flat pack and search buffers, d={d} k={k}")
+    rng = np.random.default_rng(d + k)
+    base = rng.standard_normal((4000, d)).astype(np.float32)
+    q = rng.standard_normal((5000, d)).astype(np.float32)
+    oids, odists = oracle.flat_search(base, q, k, metric=0)
+    fx = FlatIndex(d, "l2")
+    fail(2)  # rows and norms are there, the packed copy is not
+    fx.add(base)
+    fail(0, 0)
+    ids, dists = fx.search(q[:500], k)
+    assert np.array_equal(ids, oids[:500]) and dists.tobytes() == odists[:500].tobytes()
+    fx = FlatIndex(d, "l2")
+    fx.add(base)
+    # the staged queries, ids and distances, then the search buffer twice
+    fail(3, 2)
+    ids, dists = fx.search(q, k)
+    fail(0, 0)
+    assert np.array_equal(ids, oids) and dists.tobytes() == odists.tobytes()

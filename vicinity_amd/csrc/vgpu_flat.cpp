@@ -11,6 +11,8 @@ namespace vgpu {
 
 // Flagged queries the ranking path's fallback takes with the count read on the device
 constexpr size_t kFlatFallbackCap = 256;
+// The others of one launch (their keys: at most 112 MiB)
+constexpr int kFlatFallbackPass = 4096;
 
 FlatIndex::FlatIndex(size_t dim, int met) : d(dim), metric(met) {
     if (dim == 0) throw Error(VGPU_ERR_INVALID_CONFIG, "dimension must be greater than 0");
@@ -70,9 +72,17 @@ void FlatIndex::sync_device() {
         d_x.upload(host.data(), n * d, stream);
         d_xnorm.reserve(n);
         launch_flat_norms(d_x.p, (int)n, (int)d, d_xnorm.p, stream);
-        if (flat_pack_chunks((int)n, (int)d)) {
-            d_xb.reserve(flat_pack_chunks((int)n, (int)d));
-            launch_flat_pack(d_x.p, (int)n, (int)d, d_xb.p, stream);
+        // the ranking path's copy, as large as the rows: only where a search can
+        // use it, and without it the fp32 path serves every search
+        if (flat_rank_ok((int)d, 1, finite && xmax2 < 1e30)) {
+            try {
+                d_xb.reserve(flat_pack_chunks((int)n, (int)d));
+                launch_flat_pack(d_x.p, (int)n, (int)d, d_xb.p, stream);
+            } catch (const Error& e) {
+                if (e.code != VGPU_ERR_OUT_OF_MEMORY) throw;
+            }
+        } else {
+            d_xb.release();
         }
         VGPU_HIP(hipGetLastError());
         VGPU_HIP(hipStreamSynchronize(stream));
@@ -93,7 +103,16 @@ void FlatIndex::search_device(const float* d_q, size_t nq, size_t k, int64_t* d_
         return;
     }
     const bool rank = d_xb.n && flat_rank_ok((int)d, (int)k, finite && xmax2 < 1e30);
-    const size_t step = rank && k > 32 ? (size_t)flat_rank_chunk() : nq;
+    size_t step = rank && k > 32 ? std::min(nq, (size_t)flat_rank_chunk()) : nq;
+    for (;;) {  // the largest buffer; the ranking path needs more of it per query
+        try {
+            w_partial.reserve(flat_partial_count((int)step, (int)n, (int)k, rank));
+            break;
+        } catch (const Error& e) {
+            if (e.code != VGPU_ERR_OUT_OF_MEMORY || !rank || step <= 1024) throw;
+            step = (step + 1) / 2;
+        }
+    }
     float gemm = 0.f, total = 0.f;
     unsigned int fb = 0;
     for (size_t q0 = 0; q0 < nq; q0 += step) {
@@ -150,10 +169,11 @@ void FlatIndex::search_pass(const float* d_q, size_t nq, size_t k, bool rank, in
     VGPU_HIP(hipGetLastError());
     VGPU_HIP(hipStreamSynchronize(s));
     if (rsl && fallbacks > (unsigned int)cap) {  // more than the device-driven pass took
-        const int rest = (int)fallbacks - cap;
-        w_fbkeys.reserve((size_t)rest * rsl * k);
-        launch_flat_rank_fallback(w_flag.p + cap, rest, w_fb.p, w_partial.p, (int)nq, (int)n, (int)d, (int)k,
-                                  metric, d_q, d_x.p, w_fbkeys.p, w_idx.p, w_dist.p, s);
+        const int all = (int)fallbacks;
+        w_fbkeys.reserve((size_t)std::min(all - cap, kFlatFallbackPass) * rsl * k);
+        for (int f0 = cap; f0 < all; f0 += kFlatFallbackPass)
+            launch_flat_rank_fallback(w_flag.p + f0, std::min(all - f0, kFlatFallbackPass), w_fb.p, w_partial.p, (int)nq,
+                                      (int)n, (int)d, (int)k, metric, d_q, d_x.p, w_fbkeys.p, w_idx.p, w_dist.p, s);
         launch_finalize(w_idx.p, w_dist.p, nullptr, (int)nq, (int)k, (int)k, d_ids, d_dists, s);
         VGPU_HIP(hipEventRecord(ev[2], s));
         VGPU_HIP(hipGetLastError());
