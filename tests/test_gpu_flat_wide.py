@@ -102,3 +102,21 @@ def test_flat_wide_query_that_is_not_finite(oracle):
     _check(ids[rest], dists[rest], oids[rest], odists[rest])
     assert np.isnan(dists[3]).all() and np.unique(ids[3]).size == k
     assert np.isinf(dists[11]).all() and np.array_equal(ids[11], np.arange(k))
+
+
+@pytest.mark.parametrize("offset,metric,lost", [(0.5, 0, False), (3.0, 0, True), (30.0, 0, False), (12.0, 1, True)])
+def test_flat_wide_rows_far_from_the_origin(oracle, offset, metric, lost):
+    """Rows whose common offset swallows the ranking path's bound but not the
+    fp32 path's (lost): the fp32 path, which proves nearly every query; the
+    ranking path's exhaustive fallback had all of them."""
+    print(f"[case] flat wide offset {offset} metric {metric}", flush=True)
+    rng = np.random.default_rng(11)
+    n, d, k = 6000, 200, 10
+    c = rng.standard_normal((20, d))
+    c /= np.linalg.norm(c, axis=1, keepdims=True)
+    base = (c[rng.integers(0, 20, n)] + 0.05 * rng.standard_normal((n, d)) + offset).astype(np.float32)
+    q = (c[rng.integers(0, 20, 200)] + 0.05 * rng.standard_normal((200, d)) + offset).astype(np.float32)
+    fx = _index(d, metric, base)
+    _check(*fx.search(q, k), *oracle.flat_search(base, q, k, metric=metric))
+    if lost:
+        assert fx.last_fallbacks() <= 20

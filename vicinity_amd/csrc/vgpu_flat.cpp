@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "vgpu_bounds.h"
 #include "vgpu_runtime.h"
 
 namespace vgpu {
@@ -17,6 +18,7 @@ constexpr int kFlatFallbackPass = 4096;
 FlatIndex::FlatIndex(size_t dim, int met) : d(dim), metric(met) {
     if (dim == 0) throw Error(VGPU_ERR_INVALID_CONFIG, "dimension must be greater than 0");
     if (met != 0 && met != 1) throw Error(VGPU_ERR_INVALID_CONFIG, "metric must be 0 (L2) or 1 (1 - dot)");
+    rowsum.assign(d, 0.0);
     VGPU_HIP(hipStreamCreate(&stream));
     for (auto& e : ev) VGPU_HIP(hipEventCreate(&e));
 }
@@ -33,6 +35,8 @@ void FlatIndex::add(const float* x, size_t count) {
     const size_t n0 = n;
     const double xmax0 = xmax2;
     const bool finite0 = finite;
+    const std::vector<double> rowsum0 = rowsum;
+    const double sqsum0 = sqsum;
     host.insert(host.end(), x, x + count * d);
     double sum = 0.0;
     for (size_t i = 0; i < count; i++) {
@@ -45,7 +49,9 @@ void FlatIndex::add(const float* x, size_t count) {
         const double t = (p[0] + p[1]) + (p[2] + p[3]);
         xmax2 = std::max(xmax2, t);
         sum += t;
+        for (j = 0; j < d; j++) rowsum[j] += r[j];
     }
+    sqsum += sum;
     finite = finite && std::isfinite(sum);  // squares of floats: no overflow in double
     n += count;
     try {
@@ -57,6 +63,8 @@ void FlatIndex::add(const float* x, size_t count) {
         n = n0;
         xmax2 = xmax0;
         finite = finite0;
+        rowsum = rowsum0;
+        sqsum = sqsum0;
         try {
             sync_device();
         } catch (...) {
@@ -90,6 +98,26 @@ void FlatIndex::sync_device() {
     stale = false;
 }
 
+// Whether the ranking path's bf16x3 bound is lost in the rows' common offset
+// while the fp32 path's is not.  Distances are spread over about the rows'
+// variance (dot products over the norm times a dimension's deviation); where
+// the bound reaches half of that, a good part of the vectors are within it of
+// the k-th and every query ends in the exhaustive fallback, in either path.
+// 100k x 200 around unit centres plus 2, 2.5 and 3 in every dimension, k 10, 1000
+// queries: fp32 5.3 ms each, ranking path 0.6, 10.5 and 10.6; plus 10, where both
+// bounds are lost: 16.3 and 10.6.  Up to 96 dimensions the fallback is the
+// cheaper one (100k x 32, k 40: fp32 8.2 ms, ranking path 2.6, all in fallback).
+bool FlatIndex::rank_bound_lost() const {
+    if (d <= 96) return false;
+    double mean2 = 0.0;
+    for (double x : rowsum) mean2 += (x / n) * (x / n);
+    const double var = std::max(sqsum / n - mean2, 0.0), norm = std::sqrt(xmax2);
+    const double spread = metric == 0 ? var : norm * std::sqrt(var / d);
+    const float xn = (float)norm;
+    const double fp32 = 4.0 * (d + 8.0) * 5.9604645e-08 * (metric == 0 ? 4.0 * xmax2 : 1.0 + xmax2);
+    return flat_bf16_tau((int)d, metric, xn, xn, 0) > 0.5 * spread && fp32 < 0.5 * spread;
+}
+
 void FlatIndex::search_device(const float* d_q, size_t nq, size_t k, int64_t* d_ids, float* d_dists,
                               hipStream_t s) {
     if (!s) s = stream;
@@ -102,7 +130,8 @@ void FlatIndex::search_device(const float* d_q, size_t nq, size_t k, int64_t* d_
         VGPU_HIP(hipStreamSynchronize(s));
         return;
     }
-    const bool rank = d_xb.n && flat_rank_ok((int)d, (int)k, finite && xmax2 < 1e30);
+    const bool rank = d_xb.n && flat_rank_ok((int)d, (int)k, finite && xmax2 < 1e30) &&
+                      ((d <= 128 && k <= 32) || !rank_bound_lost());
     size_t step = rank && k > 32 ? std::min(nq, (size_t)flat_rank_chunk()) : nq;
     for (;;) {  // the largest buffer; the ranking path needs more of it per query
         try {

@@ -309,6 +309,8 @@ struct FlatIndex {
     std::vector<float> host;
     double xmax2 = 0.0;  // max ||x||^2
     bool finite = true;  // no row holds a NaN or an infinity
+    std::vector<double> rowsum;  // [d] sum of the rows
+    double sqsum = 0.0;          // sum of ||x||^2
     float ms_gemm = 0.f, ms_total = 0.f;
     unsigned int fallbacks = 0;  // queries of the last search that took the exhaustive exact scan
     bool stale = false;  // a failed add could not restore the device copy of the n rows
@@ -323,6 +325,7 @@ struct FlatIndex {
                        hipStream_t s);
 
   private:
+    bool rank_bound_lost() const;
     // One pass: the ranking path's (rank) queries are bounded by flat_rank_chunk.
     void search_pass(const float* d_q, size_t nq, size_t k, bool rank, int64_t* d_ids, float* d_dists,
                      hipStream_t s);
