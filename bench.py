@@ -11,8 +11,10 @@ A step is one search over the whole 10k-query batch with the queries
 already resident in HBM.  The dominant kernel is the ADC scan (the flat
 GEMM for `flat`); its duration comes from hipEvents recorded on the search's
 stream around that kernel in every timed step, and its algorithmic bytes are
-(code bytes + 4) per scanned list entry, counted by the kernel itself.  The
-CPU baseline is the oracle (the C restatement of the reference search) on the
+(code bytes + 4) per scanned list entry, counted by the kernel itself.  Where
+the batch takes the scan by inverted list, which reads a list once for many
+queries, the time is that of all its kernels and the rate is of its matrix
+products.  The CPU baseline is the oracle (the C restatement of the reference search) on the
 host cores, over a bounded sample of the same queries and index arrays.
 Recall@k is measured against exact cosine ground truth (the flat GPU path on
 the normalised vectors, the reference's own ground truth).
@@ -38,6 +40,7 @@ METRIC = "IVF-PQ QPS @ fixed nprobe, 1M×d128 batch 10k; ADC-scan HBM GB/s vs pe
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
 BF16_PEAK_TFLOPS = 2500.0
+INT8_PEAK_TOPS = 5000.0
 
 
 def log(msg):
@@ -252,10 +255,9 @@ def run_ivfpq(args, w):
     exact = args.opq or args.mode == "exact"
     route = ctypes.c_int(0)
     v._lib.check(v._lib.load().vgpu_test_scan_route(ix._h, nq, k, nprobe, pool or 0, ctypes.byref(route)))
-    if route.value:
-        # the whole scan by inverted list (pairs, sample, scores, rescoring) is
-        # timed as one; the score kernel is its largest part
-        kernel, kname = ("fs_list_kernel" if K == 16 else "list_score_kernel"), "scan_list"
+    kname = None
+    if route.value:  # pairs, sample, scores and rescoring are timed as one
+        kernel = ("fs_list_kernel" if K == 16 else "list_score_kernel") + " and the scan's other kernels"
     elif K == 16:
         kernel, kname = "fastscan_kernel", "fastscan"
     elif exact:
@@ -273,14 +275,31 @@ def run_ivfpq(args, w):
     metric = METRIC if args.workload == "ivfpq_1m" else (
         f"IVF-PQ QPS @ fixed nprobe, {w.name} batch {nq // 1000}k; ADC-scan HBM GB/s vs peak")
     line = base_line(args, metric, qps, "queries/s", ms_step, "f32", config)
+    if route.value:
+        # The scan by list reads a list once for up to 64 queries, so bytes per
+        # scored entry are not what it moves; it is held to the products it makes
+        # of them: three bf16 terms per padded dimension, or 16 one-hot int8
+        # positions per codebook.  (entry_gbs: entries times their code bytes over
+        # the same time, the figure a scan that reads every entry would need.)
+        width = d // M
+        pad = width if width <= 2 else 4 if width <= 4 else 8 * ((width + 7) // 8)
+        ops = 2 * 16 * 4 * ((M + 3) // 4) if K == 16 else 2 * 3 * 32 * ((M * pad + 31) // 32)
+        peak = INT8_PEAK_TOPS if K == 16 else BF16_PEAK_TFLOPS
+        rate = cands * ops / (scan_ms * 1e-3) / 1e12
+        roofline = {"bound": "mfma", "achieved": round(rate, 1), "peak": peak,
+                    "unit": "TOP/s" if K == 16 else "TFLOP/s", "frac": round(rate / peak, 4), "traffic": None,
+                    "kernel": kernel, "kernel_ms": round(scan_ms, 4), "table_prepass_ms": 0.0,
+                    "entry_gbs": round(achieved, 1), "candidates_per_launch": int(cands)}
+    else:
+        roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+                    "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                    "traffic": None if exact or args.n else traffic_from_profile(f"{kname}_{w.name}"),
+                    "kernel": kernel, "kernel_ms": round(scan_ms, 4),
+                    "table_prepass_ms": round(table_ms, 4),
+                    "algorithmic_bytes_per_launch": int(scan_bytes),
+                    "candidates_per_launch": int(cands)}
     line.update({
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": None if exact or args.n else traffic_from_profile(f"{kname}_{w.name}"),
-                     "kernel": kernel, "kernel_ms": round(scan_ms, 4),
-                     "table_prepass_ms": round(table_ms, 4),
-                     "algorithmic_bytes_per_launch": int(scan_bytes),
-                     "candidates_per_launch": int(cands)},
+        "roofline": roofline,
         "recall_at_k": recall,
         "phases_ms": phases,
         "fallback_queries": fallbacks,
