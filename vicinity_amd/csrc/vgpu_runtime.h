@@ -309,8 +309,9 @@ struct FlatIndex {
     std::vector<float> host;
     double xmax2 = 0.0;  // max ||x||^2
     bool finite = true;  // no row holds a NaN or an infinity
-    std::vector<double> rowsum;  // [d] sum of the rows
-    double sqsum = 0.0;          // sum of ||x||^2
+    std::vector<double> rowsum;  // [d] sum of every 16th row (above 96 dimensions),
+    double sqsum = 0.0;          // their sum of ||x||^2
+    size_t sampled = 0;          // and their number
     float ms_gemm = 0.f, ms_total = 0.f;
     unsigned int fallbacks = 0;  // queries of the last search that took the exhaustive exact scan
     bool stale = false;  // a failed add could not restore the device copy of the n rows
