@@ -86,3 +86,52 @@ def test_device_searches_on_separate_torch_streams():
     ids = torch.cat([outs[0][0], outs[1][0]]).cpu().numpy()
     d = torch.cat([outs[0][1], outs[1][1]]).cpu().numpy()
     assert np.array_equal(ids, ref_ids) and d.tobytes() == ref_d.tobytes()
+
+
+@pytest.mark.parametrize("d,M,K", [(64, 16, 256), (50, 25, 256), (32, 16, 16)])
+def test_scans_by_list_on_threads_and_streams(oracle, d, M, K):
+    """Large batches of one handle at once, each on the scan by inverted list:
+    host batches on four threads, device batches on two torch streams."""
+    import torch
+    from test_gpu_list_scan import _index, _route
+
+    _print_case(f"concurrent scans by list, d={d} M={M} ksub={K}")
+    rng = np.random.default_rng(d + K)
+    ix, oix, x = _index(oracle, rng, 4000, d, 16, M, K)
+    batches = []
+    for i in range(8):
+        nq = int(rng.integers(300, 1500))
+        q = (x[rng.integers(0, 4000, nq)] + 0.1 * rng.standard_normal((nq, d))).astype(np.float32)
+        batches.append((q, *[(10, 8), (100, 16)][i % 2]))
+    want = [oix.search_batch(*b) for b in batches]
+    assert all(_route(ix, len(q), k, P) == 1 for q, k, P in batches)
+    dev = [torch.from_numpy(q).to("cuda:0") for q, _, _ in batches]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    errors = []
+
+    def check(i, ids, dists):
+        assert np.array_equal(ids, want[i][0]) and dists.tobytes() == want[i][1].tobytes(), i
+
+    def worker(t):
+        try:
+            for _ in range(3):
+                for i in range(t % 4, len(batches), 4):
+                    q, k, P = batches[i]
+                    if t < 4:
+                        check(i, *ix.batch_search(q, k, nprobe=P))
+                        continue
+                    with torch.cuda.stream(streams[t - 4]):
+                        ids, dists = ix.search_batch_device(dev[i], k, nprobe=P, stream=streams[t - 4])
+                        streams[t - 4].synchronize()
+                        check(i, ids.cpu().numpy(), dists.cpu().numpy())
+        except Exception as e:  # surfaced in the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=120)
+    assert not any(t.is_alive() for t in threads), "a search thread did not finish"
+    assert not errors, errors

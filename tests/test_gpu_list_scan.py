@@ -220,12 +220,29 @@ def test_crowds_of_flagged_queries(oracle, opq, d, M, K):
         assert ix.last_stats()["fallback_queries"] >= 200
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,K", [(64, 256), (96, 100), (100, 256)])
+def test_one_dimensional_codebooks_of_several_steps(oracle, d, K):
+    """Two to four 32-dimension steps of one-dimensional codebooks (25, one
+    step, is among test_padded_shapes)."""
+    _print_case(f"list scan: d=M={d} ksub={K}")
+    rng = np.random.default_rng(d)
+    ix, oix, x = _index(oracle, rng, 3000, d, 12, d, K)
+    q = (x[rng.integers(0, 3000, 700)] + 0.2 * rng.standard_normal((700, d))).astype(np.float32)
+    for k, P in [(10, 9), (100, 12)]:
+        _same(ix, oix, q, k, P)
+
+
 @pytest.mark.parametrize("d,M,scale", [(32, 8, 1.0), (96, 48, 0.05), (128, 16, 30.0)])
 def test_error_bound(oracle, d, M, scale):
-    """|a - e| <= list_tau with a from bf16x3 products in float32 (started
-    from -|y|^2 / 2, summed in order or truncated) and e the reference's
-    float32 distance; without its product term the bound fails."""
-    from test_proof_bounds import bf16_split, seq_sum
+    """|a - e| <= list_tau with a from bf16x3 products as the score kernel makes
+    them (32-dimension steps, low times high, high times low, high times high,
+    started from -|y|^2 / 2; each step's sum rounded once, after every product, or
+    toward zero) and e the reference's float32 distance.  Random residuals, and
+    rows whose low halves are largest and of one sign: there the products dropped
+    from bf16x3 alone exceed the bound's other terms."""
+    from test_flat_key_bound import _score
+    from test_proof_bounds import seq_sum
 
     from vicinity_amd import _lib
 
@@ -233,21 +250,24 @@ def test_error_bound(oracle, d, M, scale):
     F32 = np.float32
     r = (scale * rng.standard_normal((200, d))).astype(F32)
     y = (r + scale * 10.0 ** rng.uniform(-3, 0, (200, 1)) * rng.standard_normal((200, d))).astype(F32)
+    r[:20] = y[:20] = 2.0 ** np.round(np.log2(scale)) * (1.0 + 2.0 ** -8 * rng.uniform(0.97, 0.999, (20, d)))
     yn = np.sum(y.astype(np.float64) ** 2, 1)
-    rh, rl = bf16_split(r)
-    yh, yl = bf16_split(y)
-    terms = np.concatenate([(-0.5 * yn).astype(F32)[:, None], yh * rl, yl * rh, yh * rh], 1).astype(F32)
     t0 = seq_sum((r * r).astype(F32))
     diff = (r - y).astype(F32)
-    e = seq_sum(seq_sum((diff * diff).astype(F32).reshape(200, M, -1)))
+    e = seq_sum(seq_sum((diff * diff).astype(F32).reshape(200, M, -1))).astype(np.float64)
     out = ctypes.c_float()
-    worst = 0.0
+    tau, rest = np.empty(200), np.empty(200)
+    u, ds = 2.0 ** -24, d // M
     for i in range(200):
-        D = seq_sum(terms[i:i + 1])[0]
-        a = F32(np.float64(t0[i]) - 2.0 * np.float64(D))
-        _lib.check(_lib.load().vgpu_test_bound_list(d, M, d // M, float(t0[i]), float(np.sqrt(yn[i])),
+        _lib.check(_lib.load().vgpu_test_bound_list(d, M, ds, float(t0[i]), float(np.sqrt(yn[i])),
                                                     ctypes.byref(out)))
-        err = abs(float(a) - float(e[i]))
-        assert err <= out.value, (i, err, out.value)
-        worst = max(worst, err / out.value)
-    assert worst > 1e-3  # the inputs come within reach of the bound
+        tau[i] = out.value
+        # the terms that are not the products'
+        rest[i] = 1.25 * ((d + 4) * u * t0[i] + (ds + M + 6) * u * (np.sqrt(t0[i]) + np.sqrt(yn[i])) ** 2)
+    for order in ("exact", "seq", "trunc"):
+        D = _score(y, r, (-0.5 * yn).astype(F32), order).astype(np.float64)
+        a = (t0.astype(np.float64) - 2.0 * D).astype(F32)  # one rounding, as the kernel's fma
+        err = np.abs(a.astype(np.float64) - e)
+        assert (err <= tau).all(), (order, (err / tau).max())
+        assert (err[:20] > rest[:20]).all(), (order, (err[:20] / rest[:20]).min())
+        assert (err / tau).max() > 0.05, (order, (err / tau).max())
