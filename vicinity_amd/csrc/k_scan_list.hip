@@ -15,7 +15,9 @@
 //       every list, and the work items (a list's segment x up to 64 of its
 //       pairs) the score kernel's waves take in turn.
 //   list_score_kernel<.., SAMPLE>   the first 16 TCAP entries of each query's
-//       nearest lists: an upper bound of every entry's distance.
+//       nearest lists: an upper bound of every entry's distance.  TCAP is 32 to
+//       256 by the rule in vgpu_index.cpp: the longer the lists and the larger
+//       k, the more entries the bound of a small sample leaves.
 //   list_bound_kernel     the k-th smallest of those bounds, which bounds the
 //       query's k-th distance from above.
 //   list_score_kernel<.., !SAMPLE>  every pair: entries whose distance may be
@@ -33,15 +35,16 @@
 // list_rescue_kernel, or for many of them the EXACT kernel, scores its entries
 // with the reference's arithmetic.
 //
-// Bounds, at 10k queries: the score kernel is held by the LDS codeword gathers
-// and the latency of the work items' prologues, at two waves per SIMD (the
-// operands of 64 pairs fill the registers): 125 us for 76M entries of 128
-// dimensions (matrix cores busy 30 us), 380 us for 390M of 96, 165 us for 370M
-// of 25.  The final kernel is held by the L1 line rate of its codeword loads
-// (108 us for 102 rescored entries per query, 16 codebooks of 8).  The whole
-// scan against the kernels it replaces: 1M x 128 331 -> 305 us (FAST scan and
-// its tables), 10M x 96 3400 -> 640, 1.2M x 25 2520 -> 290, OPQ 500k x 128 (5k
-// queries) 833 -> 205.
+// Bounds, at 10k queries: the score kernel is held by latency, of the decode's
+// LDS gathers and of the work items' prologues, at two waves per SIMD (the
+// operands of 64 pairs fill the registers).  126 us for 76M entries of 128
+// dimensions: matrix cores 22% busy, VALU 30%, LDS 20% (half of it bank
+// conflicts), waves waiting 45% of their time; 390 us for 390M of 96, 166 us for
+// 370M of 25.  The final kernel is held by its codeword loads (109 us for 102
+// rescored entries per query, 16 codebooks of 8: L1 64% of its cycles, VALU 54%,
+// waves waiting 65%).  The whole scan against the kernels it replaces, traced: 1M
+// x 128 331 -> 317 us (FAST scan and its tables), 10M x 96 3400 -> 726, 1.2M x 25
+// 2520 -> 292, OPQ 500k x 128 (5k queries) 833 -> 199.
 //
 // MFMA layout (wave64): lane l holds row / column l % 16 and the eight
 // dimensions 8 (l / 16) .. + 7 of a 32-dimension step, for A (entries) and B
@@ -1082,6 +1085,7 @@ template <int DS>
 __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs a, ListWs w) {
     extern __shared__ __align__(16) char smem[];
     __shared__ uint32_t cnt, last;
+    __shared__ uint64_t bound;
     const uint32_t nf = *a.flag_count;
     if (nf == 0 || nf > SL_RESCUE_MAX) return;
     uint64_t* keys = reinterpret_cast<uint64_t*>(smem);
@@ -1089,8 +1093,7 @@ __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs 
     float* r = reinterpret_cast<float*>(smem + SL_TOP * 8);  // [d]
     uint32_t* sl_l = reinterpret_cast<uint32_t*>(r + (d + 3) / 4 * 4);  // [P] lists, first positions, lengths
     uint32_t *sl_o = sl_l + a.P, *sl_n = sl_o + a.P;
-    // workgroups per query; their keys are merged in one sort
-    const uint32_t S = min(min(64u, SL_RESCUE / nf), max(8u, (SL_TOP - 2 * VGPU_BLOCK) / (uint32_t)k));
+    const uint32_t S = min(64u, SL_RESCUE / nf);  // workgroups per query: 8 to 64
     for (uint32_t job = blockIdx.x; job < nf * S; job += gridDim.x) {
         const uint32_t f = job / S, sl = job % S, q = a.flag_list[f];
         const uint32_t* pr = a.probe + (size_t)q * a.P;
@@ -1159,9 +1162,24 @@ __global__ __launch_bounds__(256) void list_rescue_kernel(DevIndex ix, ScanArgs 
         __syncthreads();
         if (!last) continue;
         __threadfence();
-        if (tid == 0) cnt = 0u;
-        top.thr = ~0ull;
+        // Every workgroup has (k - 1) / S + 1 keys up to the largest of their keys of
+        // that rank, together at least k: keys above it are out (6400 keys of 64
+        // workgroups at k 100 were four sorts of the buffer, 80 us).
+        if (tid < 64) {
+            uint64_t t = tid < S ? __hip_atomic_load(part + (size_t)tid * k + (k - 1) / S, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)
+                                 : 0ull;
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint64_t x = (uint64_t)__shfl_xor((long long)t, o, 64);
+                t = x > t ? x : t;
+            }
+            if (tid == 0) {
+                cnt = 0u;
+                bound = t;
+            }
+        }
         __syncthreads();
+        top.thr = bound == ~0ull ? ~0ull : bound + 1ull;
         for (uint32_t b = 0; b < S * (uint32_t)k; b += VGPU_BLOCK) {
             const bool ok = b + tid < S * (uint32_t)k;
             const uint64_t key =
