@@ -29,13 +29,14 @@
 // 16-byte read of the nibble's one-hot row from LDS.  Each codeword that is
 // read from LDS serves both tiles.
 //
-// Bounds, at 10k queries x 64 lists of 488 entries, M 50: the table build's
-// vector instructions and LDS reads (two passes over 800 values per pair, as in
-// fastscan_kernel), then the one-hot reads; the matrix cores are busy about
-// 100 of 830 us.  Whole search 2730 -> 1117 us.  The rows' parts of the next
-// step are loaded under the present one (1313 -> 1253), and items hold 32
-// pairs, one pass of a wave: with 64 the few popular lists' waves ran twice as
-// long at the end of the sample and of the scan (1253 -> 1117).
+// Bounds, at 10k queries x 64 lists of 488 entries, M 50: the vector
+// instructions, most of them the table build's (two passes over 800 values per
+// pair, as in fastscan_kernel).  VALU 62% busy, matrix cores 16% (115 us), LDS
+// 14%, waves waiting 43% of their time, in the 738 us of the scan; the sample
+// takes 144.  Whole search 2718 -> 1117 us.  The rows' parts of the next step
+// are loaded under the present one (1313 -> 1253), and items hold 32 pairs, one
+// pass of a wave: with 64 the few popular lists' waves ran twice as long at the
+// end of the sample and of the scan (1253 -> 1117).
 #include "vgpu_device.h"
 #include "vgpu_launch.h"
 
