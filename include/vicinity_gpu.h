@@ -71,11 +71,13 @@ typedef struct vgpu_search_stats {
     float ms_normalize, ms_coarse, ms_select, ms_scan, ms_fallback, ms_rerank, ms_total;
     uint64_t candidates;     /* sum over queries of scanned list entries */
     uint64_t scan_bytes;     /* algorithmic bytes of the scan: candidates * (code bytes + 4) */
-    uint32_t fallback_queries; /* FAST queries recomputed in EXACT mode */
+    uint32_t fallback_queries; /* FAST queries recomputed in EXACT mode; scan by inverted list: queries
+                                * whose survivors could not all be ranked (their time is in ms_scan) */
     uint32_t coarse_overflow;  /* queries whose probe selection took the exact fallback */
     uint32_t nq;
     uint64_t fast_flushes;     /* FAST: buffer flushes summed over queries */
-    uint64_t fast_appends;     /* FAST: entries that passed the running threshold */
+    uint64_t fast_appends;     /* FAST: entries that passed the running threshold; scan by inverted
+                                * list: entries within the sample's bound */
     uint32_t fallback_ties;    /* FAST fallbacks caused by more equal distances than the buffer holds */
     uint32_t fast_retries;     /* FAST queries that needed a second pass over their lists */
     float ms_table;            /* FAST: the per-query table pre-pass (not part of ms_scan) */
