@@ -50,11 +50,15 @@ void FlatIndex::add(const float* x, size_t count) {
         const double t = (p[0] + p[1]) + (p[2] + p[3]);
         xmax2 = std::max(xmax2, t);
         sum += t;
-        if (d > 96 && (n0 + i) % 16 == 0) {  // rank_bound_lost: a sample is enough
-            for (j = 0; j < d; j++) rowsum[j] += r[j];
-            sqsum += t;
-            sampled++;
+    }
+    for (size_t i = (16 - n0 % 16) % 16; d > 96 && i < count; i += 16, sampled++) {  // rank_bound_lost
+        const float* r = x + i * d;
+        double t = 0.0;
+        for (size_t j = 0; j < d; j++) {
+            rowsum[j] += r[j];
+            t += (double)r[j] * r[j];
         }
+        sqsum += t;
     }
     finite = finite && std::isfinite(sum);  // squares of floats: no overflow in double
     n += count;
