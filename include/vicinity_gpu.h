@@ -330,9 +330,10 @@ int vgpu_test_bound_list(size_t padded_d, size_t M, size_t ds, float t0, float y
  * scan by inverted list (a test hook; no device call). */
 int vgpu_test_scan_route(vgpu_ivfpq *h, size_t nq, size_t k, size_t nprobe, size_t rerank_pool, int *out);
 /* The rule behind it for an index of n entries in L lists: sample tiles per
- * query of the scan by inverted list, 0 the mode's own scan. */
+ * query of the scan by inverted list, 0 the mode's own scan (repeats: entries
+ * of a list that share an entry's codes, on average). */
 int vgpu_test_list_rule(size_t d, size_t M, size_t K, size_t L, size_t n, size_t nq, size_t P, size_t k, int opq,
-                        int *out);
+                        float repeats, int *out);
 /* always != 0: every batch search whose shape has the scan by inverted list
  * takes it, also where the rule prefers the mode's own scan. */
 int vgpu_test_set_list_scan(vgpu_ivfpq *h, int always);

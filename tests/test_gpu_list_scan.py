@@ -126,11 +126,11 @@ def test_equal_distances_beyond_the_buffers(oracle, copies, k):
     assert ix.last_stats()["fallback_queries"] >= 40
 
 
-def _rule(d, M, K, L, n, nq, P, k, opq=0):
+def _rule(d, M, K, L, n, nq, P, k, opq=0, repeats=1.0):
     from vicinity_amd import _lib
 
     out = ctypes.c_int(-1)
-    _lib.check(_lib.load().vgpu_test_list_rule(d, M, K, L, n, nq, P, k, opq, ctypes.byref(out)))
+    _lib.check(_lib.load().vgpu_test_list_rule(d, M, K, L, n, nq, P, k, opq, repeats, ctypes.byref(out)))
     return out.value
 
 
@@ -139,6 +139,8 @@ def _rule(d, M, K, L, n, nq, P, k, opq=0):
     (128, 16, 256, 256, 1_000_000, 1000, 64, 100, 0), (128, 16, 256, 16, 300_000, 1000, 8, 100, 0),
     (128, 16, 256, 1, 300_000, 500, 1, 10, 0), (128, 16, 256, 2, 300_000, 500, 2, 10, 0),
     (128, 16, 256, 64, 300_000, 1000, 64, 100, 0), (128, 16, 256, 16, 300_000, 5000, 8, 100, 1),
+    # few entries per query: the FAST scan has little to do
+    (32, 8, 256, 1024, 50_000, 4000, 20, 10, 0), (128, 16, 256, 1024, 300_000, 16_000, 1, 100, 0),
     (100, 50, 16, 1, 300_000, 500, 1, 100, 0), (100, 50, 16, 8, 300_000, 500, 4, 100, 0),
     # rescoring by odd widths costs more than the lookups saved
     (96, 16, 256, 1024, 300_000, 10_000, 32, 100, 0), (96, 32, 256, 1024, 300_000, 10_000, 32, 200, 0),
@@ -164,6 +166,26 @@ def test_rule_takes_the_scan_by_list(d, M, K, L, n, nq, P, k, opq, tiles):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [16, 12])
+def test_rotated_entries_that_share_codes(oracle, M):
+    """An OPQ index whose lists hold many copies of few code rows: its batches
+    keep the EXACT scan, which has no ties to fail on; copies of no row: they do
+    not."""
+    rng = np.random.default_rng(M)
+    d = M * 8
+    rot = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((d, d)))[0].astype(np.float32))
+    for distinct, route in [(12, 0), (6000, 1)]:
+        _print_case(f"list scan: OPQ M={M}, {distinct} distinct rows of 30,000")
+        x = rng.standard_normal((distinct, d)).astype(np.float32)[rng.integers(0, distinct, 30_000)]
+        if route:  # near copies: codes of their own
+            x += 0.3 * rng.standard_normal(x.shape).astype(np.float32)
+        ix, oix, xn = _index(oracle, rng, len(x), d, 12, M, 256, rotation=rot, x=x)
+        _always(ix, 0)
+        q = (x[rng.integers(0, len(x), 2000)] + 1e-3 * rng.standard_normal((2000, d))).astype(np.float32)
+        _same(ix, oix, q, 10, 12, route=route)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,tiles", [(9000, 64), (25_000, 128), (50_000, 256)])
 def test_larger_samples(oracle, n, tiles):
     _print_case(f"list scan: samples of {tiles} tiles")
@@ -179,22 +201,23 @@ def test_larger_samples(oracle, n, tiles):
 @pytest.mark.gpu
 @pytest.mark.parametrize("opq", [False, True])
 def test_unclustered_rows_in_few_long_lists(oracle, opq):
-    """Uniform rows, two lists, k 100: with the scan by list nearly every query
-    left more survivors than its buffer holds.  The mode's own scan is taken,
+    """Uniform rows, six lists, k 250: with the scan by list nearly every query
+    leaves more survivors than its buffer holds, whatever
+    its sample.  The mode's own scan is taken,
     and the scan by list still agrees."""
-    _print_case(f"list scan: uniform rows in two lists, opq {opq}")
+    _print_case(f"list scan: uniform rows in six lists, opq {opq}")
     rng = np.random.default_rng(8)
-    n, d = 40_000, 32
+    n, d = 80_000, 32
     x = rng.random((n, d)).astype(np.float32)
     rot = np.ascontiguousarray(np.linalg.qr(rng.standard_normal((d, d)))[0].astype(np.float32)) if opq else None
     ix, oix, _ = _index(oracle, rng, n, d, 6, 8, 256, rotation=rot, x=x)
     q = rng.random((200, d)).astype(np.float32)
-    _same(ix, oix, q, 100, 6)
+    _same(ix, oix, q, 250, 6)
     assert ix.last_stats()["fallback_queries"] > 64  # more than list_rescue_kernel takes
-    _same(ix, oix, q[:20], 100, 6)
+    _same(ix, oix, q[:20], 250, 6)
     assert 0 < ix.last_stats()["fallback_queries"] <= 64
     _always(ix, 0)
-    _same(ix, oix, q, 100, 6, route=0)
+    _same(ix, oix, q, 250, 6, route=0)
 
 
 @pytest.mark.gpu

@@ -152,7 +152,7 @@ SIGNATURES = {
     "vgpu_test_fail_device_allocations": (_i, [_sz, _sz]),
     "vgpu_test_bound_list": (_i, [_sz, _sz, _sz, _f, _f, _vp]),
     "vgpu_test_scan_route": (_i, [_vp, _sz, _sz, _sz, _sz, _vp]),
-    "vgpu_test_list_rule": (_i, [_sz, _sz, _sz, _sz, _sz, _sz, _sz, _sz, _ci, _vp]),
+    "vgpu_test_list_rule": (_i, [_sz, _sz, _sz, _sz, _sz, _sz, _sz, _sz, _ci, _f, _vp]),
     "vgpu_test_set_list_scan": (_i, [_H, _ci]),
     "vgpu_test_bound_fast_tau": (_i, [_sz, _sz, _sz, _f, _f, _f, _f, _vp]),
     "vgpu_test_bound_coarse": (_i, [_sz, _f, _f, _vp, _vp]),

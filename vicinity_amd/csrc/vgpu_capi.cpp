@@ -645,10 +645,10 @@ int vgpu_test_scan_route(vgpu_ivfpq* h, size_t nq, size_t k, size_t nprobe, size
 }
 
 int vgpu_test_list_rule(size_t d, size_t M, size_t K, size_t L, size_t n, size_t nq, size_t P, size_t k, int opq,
-                        int* out) {
+                        float repeats, int* out) {
     return guard([&] {
         need(out && d && M && d % M == 0 && L, VGPU_ERR_INVALID_PARAMETER, "bad argument");
-        *out = vgpu::list_scan_tiles(d, M, K, d / M, L, n, nq, P, k, opq != 0);
+        *out = vgpu::list_scan_tiles(d, M, K, d / M, L, n, nq, P, k, opq != 0, repeats);
     });
 }
 

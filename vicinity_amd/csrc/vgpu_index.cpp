@@ -632,6 +632,7 @@ void IvfpqIndex::upload_list_scan() {
     if (!(dix.cmax < 1e15f) || !(dix.rmax < 1e15f)) lshape.ok = false;
     for (float x : centroids) lshape.ok = lshape.ok && std::isfinite(x);
     for (float x : codebooks) lshape.ok = lshape.ok && std::isfinite(x);
+    code_repeats = lshape.ok && !rotation.empty() && K != 16 ? sampled_code_repeats() : 1.0;
     if (lshape.ok) {
         try {
             upload_list_arrays();
@@ -655,6 +656,31 @@ void IvfpqIndex::upload_list_scan() {
     dix.ltable = nullptr;
     dix.ltoff = nullptr;
     dix.ltiles = 0;
+}
+
+// How many entries of its list share an entry's codes, itself included, on
+// average: up to 512 entries of 64 lists.
+double IvfpqIndex::sampled_code_repeats() const {
+    double sum = 0.0, rows = 0.0;
+    std::vector<uint64_t> h;
+    for (size_t l = 0; l < L; l += std::max<size_t>(1, L / 64)) {
+        const size_t len = offsets[l + 1] - offsets[l], m = std::min<size_t>(len, 512);
+        if (m == 0) continue;
+        h.assign(m, 14695981039346656037ull);
+        for (size_t i = 0; i < m; i++) {
+            const uint8_t* c = &codes[(size_t)list_ids[offsets[l] + i * len / m] * M];
+            for (size_t j = 0; j < M; j++) h[i] = (h[i] ^ c[j]) * 1099511628211ull;  // FNV-1a
+        }
+        std::sort(h.begin(), h.end());
+        double pairs = 0.0;  // of equal rows, each row with itself among them
+        for (size_t i = 0, e; i < m; i = e) {
+            for (e = i; e < m && h[e] == h[i];) e++;
+            pairs += (double)(e - i) * (double)(e - i);
+        }
+        sum += (double)m + (pairs - (double)m) * (double)len / (double)m;
+        rows += (double)m;
+    }
+    return rows > 0.0 ? sum / rows : 1.0;
 }
 
 void IvfpqIndex::upload_list_arrays() {
@@ -794,10 +820,8 @@ vgpu_search_stats IvfpqIndex::last_stats() {
     return stats;
 }
 
-// Sample tiles (per query) of the scan by inverted list for nq queries of P
-// probes into n entries, or 0 where the mode's own scan is the better one.
-//
-// Survivors.  The sample is S = 16 tiles of the query's E entries, and the
+// Sample tiles (per query) of the scan by inverted list for P probes of n / L
+// entries, or 0.  The sample is S = 16 tiles of the query's E entries, and the
 // k-th smallest of it bounds the query's k-th distance, so k E / S entries are
 // within the bound on average and, where the sample is no better than a random
 // one, (k + 3.1 sqrt(k) + 3) E / S in one query of a thousand (the sum of k
@@ -805,17 +829,28 @@ vgpu_search_stats IvfpqIndex::last_stats() {
 // search whose largest sample leaves more than 0.85 of one keeps the other
 // scan, since every entry of a query that overflows is scored a second time.
 // Without this, 1000 queries, k 100: 1M uniform x 128, 512 lists, 32 probes
-// 443 -> 6086 us; 300k x 128, 16 lists, 8 probes 512 -> 6492.  A 4-bit query
-// that overflows is only scanned again by fastscan_kernel, and the sample is
-// of the nearest lists, so there 16 lists are counted: 300k x 100, M 50, k 100,
-// 500 queries, 1 list 2706 -> 5109 us, 8 lists and 4 probes 734 -> 1119; 64
-// lists and 64 probes 888 -> 382, uniform rows 1946 -> 1895.
-int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n, size_t nq, size_t P, size_t kout,
-                    bool opq) {
-    const double k = (double)kout, pairs = (double)nq * P, len = (double)n / L, entries = pairs * len;
+// 443 -> 6086 us (342 with 256 tiles); 300k x 128, 16 lists, 8 probes 512 ->
+// 6492.  A 4-bit query that overflows is only scanned again by fastscan_kernel,
+// and the sample is of the nearest lists, so there 16 lists are counted: 300k x
+// 100, M 50, k 100, 500 queries, 1 list 2706 -> 5109 us, 8 lists and 4 probes
+// 734 -> 1119; 64 lists and 64 probes 888 -> 382, uniform rows 1946 -> 1895.
+static int list_sample_tiles(size_t K, size_t L, size_t n, size_t P, size_t kout) {
+    const double k = (double)kout, len = (double)n / L;
     auto survivors = [&](double probes, int tiles) {
         return (k + 3.1 * std::sqrt(k) + 3.0) * probes * len / (16.0 * tiles);
     };
+    if (K == 16) return survivors(std::min<double>(P, 16), 128) <= SL_CAP16 ? 128 : 0;
+    int tiles = kout <= 128 ? 32 : 64;
+    while (tiles < 256 && survivors(P, tiles) > 0.5 * SL_CAP) tiles *= 2;
+    return survivors(P, tiles) > 0.85 * SL_CAP ? 0 : tiles;
+}
+
+// The same for nq queries, or 0 where the mode's own scan is the better one.
+int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n, size_t nq, size_t P, size_t kout,
+                    bool opq, double repeats) {
+    const double k = (double)kout, pairs = (double)nq * P, len = (double)n / L, entries = pairs * len;
+    const int tiles = list_sample_tiles(K, L, n, P, kout);
+    if (!tiles) return 0;
     if (K == 16) {
         // Cost.  The 4-bit scan by list has about 120 us of launches and sampling
         // above fastscan_kernel's and less per entry; both build a table per
@@ -826,44 +861,57 @@ int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n,
         // 224 / 340 -> 239; M 50, 488 per list, 432 -> 335 / 476 -> 364; M 64, 293
         // per list, 547 -> 404 / 626 -> 406; M 50, 136 per list, k 100, 752 -> 555.
         const bool large_k = kout >= 64;
-        if (pairs < 16.0 * L || entries < (large_k ? 25e6 : 30e6) || n < (large_k ? 96 : 256) * L) return 0;
-        return survivors(std::min<double>(P, 16), 128) <= SL_CAP16 ? 128 : 0;
+        const bool enough = pairs >= 16.0 * L && entries >= (large_k ? 25e6 : 30e6) && n >= (large_k ? 96 : 256) * L;
+        return enough ? tiles : 0;
     }
-    // up to three codebooks: the entries of a long list share codes, and the ties
-    // overflow the buffers (300k x 32, 128 lists, 1000 queries 221 -> 426 us)
-    if (pairs < 1.5 * L || (opq && M < 4 && len > 512)) return 0;
-    int tiles = kout <= 128 ? 32 : 64;
-    while (tiles < 256 && survivors(P, tiles) > 0.5 * SL_CAP) tiles *= 2;
-    if (survivors(P, tiles) > 0.85 * SL_CAP) return 0;
-    // Cost, in ns (entries in ps), as measured at 300k rows in 1024 lists (32 probes), 4096 (64)
-    // and 128 (4) over 43 shapes.  An entry of the scan by list costs its
-    // matrix product, one of the other scans M lookups, with the codebook count
-    // compiled in or not.  A result costs its rescoring, whose
-    // codewords are gathered whole where the width is 4 or 8 and float by float
-    // elsewhere; the other scans have part of it too.  The EXACT scan of an OPQ
-    // index builds a table per pair.  The scan by list has more launches, a
-    // sample, and arrays over the lists; few wide codebooks, whose code several
-    // virtual codebooks share, gather the same rows of the table at once.
+    const bool compiled = scan8_fast_compiled((int)M, (int)K);
+    // Entries of a list that share all their codes tie, and more ties than are
+    // rescored leave a query to be scanned again.  The EXACT scan of an OPQ index
+    // has no such queries: 300k x 128, 160 lists, 4 probes, 2000 queries, 16
+    // codebooks, 23 sharing entries 278 -> 287 us (one: 294 -> 199), 4 codebooks,
+    // 106 293 -> 470.  Its run-time kernel is slower: 6 codebooks, 77 565 -> 442,
+    // but 163 -> 288 at 50 queries; 2 codebooks, 229 279 -> 424.
+    if (pairs < 1.5 * L || (opq && repeats > (compiled ? 8.0 : 32.0))) return 0;
+    // Cost, in ns: what the two scans' times differ in, fitted to both sides of
+    // 1530 calls (51 shapes, 160 to 4096 lists, 1 to 64 probes, 1000 to 16,000
+    // queries, k 10 and 100; the whole times fit within 20% in nine of ten).  A
+    // FAST query has its table to fill and prove by, an entry its M lookups, with
+    // the codebook count compiled in or not; the EXACT scan of an OPQ index
+    // builds a table per pair.  In the scan by list an entry costs its matrix
+    // product and a result its rescoring, whose codewords are gathered whole
+    // where the width is 4 or 8 and float by float elsewhere.  That scan has more
+    // launches, a sample, and arrays over the lists, in every chunk; few wide
+    // codebooks, whose code several virtual codebooks share, gather the same rows
+    // of the table at once; and a wave walks a sixteenth of a list, at least (300k
+    // rows in one list, 500 queries, k 1 594 -> 994 us).  Fewer queries than the
+    // other scans run side by side take as long as that many.  5% to spare: of
+    // about 1500 calls in its reach some 20 become more than 1.08 times as long
+    // and 14 gains of more than 1.15 are left out.
     // Before, entries times codebooks alone decided: 10,000 queries, 94M
     // entries, 16 codebooks of 6, k 100 445 -> 810 us; 32 of 3, k 200 927 ->
     // 1246; 1200 queries, 8 codebooks of 32 codewords of 12 120 -> 170.
     const ListShape sh = list_shape((int)d, (int)M, (int)K, (int)ds);
-    const bool compiled = scan8_fast_compiled((int)M, (int)K);
-    const double m = (double)M, dd = (double)d;
-    const double by_code = compiled ? 1.0 + 0.17 * m : K == 256 ? 2.6 + 0.24 * m : 2.2 + 0.19 * m;
-    const double rescore = ds == 8   ? 0.04 + 0.0006 * dd
-                           : ds == 4 ? 0.07 + 0.0015 * dd
-                           : ds <= 2 ? (M > 32 && M < 64 ? 0.0075 : 0.0105) * m
-                           : ds < 8  ? 0.06 + 0.005 * dd
-                                     : 0.05 + 0.0085 * dd;
-    const double tables =
-        opq ? pairs * (compiled ? 0.03 * dd * (double)K / 256.0 + 0.05 * m - 0.5 : 20.0) : 0.0;
-    const double fixed = (opq ? 16e3 : (compiled ? 45e3 : 35e3) + 14e3 * (sh.parts - 1)) + 2.5 * (double)L;
-    // a wave walks a sixteenth of a list, at least: 300k rows in one list, 500
-    // queries, k 1 594 -> 994 us
-    const double by_list = std::max(1e-3 * entries * (0.6 + 0.25 * sh.KT), 4.5 * len);
-    const double saved = 1e-3 * entries * by_code + tables - by_list;
-    return saved > fixed + (double)nq * k * (rescore - 0.0025 * (compiled || opq ? m : dd)) ? tiles : 0;
+    const double m = (double)M, dd = (double)d, q = (double)nq, results = q * k, kt = sh.KT, kd = dd * (double)K / 256.0;
+    const double p = (double)P, e = 1e-3 * p * len;  // per query: pairs, thousands of entries
+    const double exact = compiled ? 17.0 + (0.1 + 0.033 * dd + 0.039 * m) * p + (1.9 + 0.23 * m) * e
+                                  : 13.0 + 0.33 * kd * p + 4.2 * e;
+    const double per_query =
+        opq ? exact + 4e-4 * dd * k
+        : compiled ? 2.6 + 0.28 * m + 0.06 * dd + 0.11 * p + (0.34 + 0.14 * m) * e + 0.0024 * m * k
+        : K == 256 ? 1.0 + 0.35 * m + 0.11 * dd + 0.13 * p + (1.4 + 0.23 * m) * e + (0.0028 * dd + 0.001 * m) * k
+                   : 4.5 + 0.02 * m + 0.05 * dd + 0.1 * p + 0.26 * m * e + (0.0021 * dd + 0.0015 * m) * k;
+    const double other = per_query * std::max(q, opq || compiled ? 300.0 : 600.0);
+    const double rescore = 0.06 + (ds == 8   ? 0.0004 * dd
+                                   : ds == 4 ? 0.0045 * m
+                                   : ds <= 2 ? 0.0035 * dd
+                                   : ds < 8  ? 0.0047 * dd
+                                             : 0.0075 * dd);
+    const double chunks = std::ceil(std::max(q / 16384.0, pairs / (1 << 22)));  // (plan_search)
+    const double fixed = opq ? 24e3 + 9e3 * (sh.parts - 1) + 7.0 * (double)L : 38e3 + 11.4e3 * (sh.parts - 1) + 9.4 * (double)L;
+    const double scored = opq ? (0.06 * kt + 5.4e-5 * dd * dd) * pairs + 1e-3 * (0.12 + 0.27 * kt) * entries
+                              : 0.036 * kt * pairs + 0.27e-3 * kt * entries;
+    const double by_list = chunks * fixed + (opq ? 4.0 : 4.7) * q + std::max(scored, 4.5 * len) + rescore * results;
+    return other > 1.05 * by_list ? tiles : 0;
 }
 
 // Whether a search of nq queries takes the scan by inverted list, and its
@@ -874,8 +922,9 @@ static bool use_list_scan(const IvfpqIndex& ix, size_t nq, SearchPlan& pl) {
     while (((size_t)1 << sb) < pl.P) sb++;
     pl.tbits = std::min(26, 32 - sb);
     if (ix.max_list >= (1u << pl.tbits)) return false;
-    pl.tcap = list_scan_tiles(ix.d, ix.M, ix.K, ix.ds, ix.L, ix.n(), nq, pl.P, pl.kout, pl.opq);
-    if (!pl.tcap && ix.list_always) pl.tcap = ix.K == 16 ? 128 : pl.kout <= 128 ? 32 : 64;
+    pl.tcap = list_scan_tiles(ix.d, ix.M, ix.K, ix.ds, ix.L, ix.n(), nq, pl.P, pl.kout, pl.opq, ix.code_repeats);
+    if (!pl.tcap && ix.list_always)
+        pl.tcap = std::max(list_sample_tiles(ix.K, ix.L, ix.n(), pl.P, pl.kout), ix.K == 16 ? 128 : pl.kout <= 128 ? 32 : 64);
     if (!pl.tcap) return false;
     pl.cap = ix.K == 16 ? SL_CAP16 : SL_CAP;
     pl.rcap = 256;

@@ -73,7 +73,7 @@ struct DevBuf {
 // The rule by which a search takes the scan by inverted list (its sample
 // tiles per query; 0: the mode's own scan).
 int list_scan_tiles(size_t d, size_t M, size_t K, size_t ds, size_t L, size_t n, size_t nq, size_t P, size_t kout,
-                    bool opq);
+                    bool opq, double repeats);
 
 // Sizes of one search call's device workspace: per query chunk, the
 // normalised queries, coarse candidates or score rows, probe lists, scan
@@ -181,6 +181,7 @@ struct IvfpqIndex {
     DevBuf<int> d_dimmap;
     ListShape lshape;
     uint32_t max_list = 0;          // entries of the longest list
+    double code_repeats = 1.0;      // OPQ: entries of a list that share an entry's codes, on average
     DevIndex dix;
 
     // build workspace (k-means assignment), used under the exclusive lock
@@ -291,6 +292,7 @@ struct IvfpqIndex {
     void snapshot_list_masks();
     void upload_list_scan();    // the arrays of the scan by inverted list, where it can be taken
     void upload_list_arrays();
+    double sampled_code_repeats() const;
     void refresh_categories(hipStream_t s);
 };
 
