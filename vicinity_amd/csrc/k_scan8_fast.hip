@@ -1820,9 +1820,9 @@ static int table_copies(const DevIndex& ix) {
 }
 
 // The codebook counts launch_scan8_fast fixes at compile time, with 256
-// codewords: rows of whole 16-byte or 4-byte loads that index files commonly
-// have.  Any other count takes the
-// run-time kernel, whose rows are read a byte at a time.
+// codewords: those whose rows are whole 16-byte loads, or 4 or 8 bytes, in the
+// shapes that were measured (24, 80, 112 and 128 were not).  Any other count
+// takes the run-time kernel, which reads a row a byte at a time.
 bool scan8_fast_compiled(int M, int K) {
     return K == 256 && (M == 4 || M == 8 || M == 16 || M == 32 || M == 48 || M == 64 || M == 96);
 }
